@@ -203,7 +203,7 @@ int matmul_bf16(scry_buf a, scry_buf b, int m, int k, int n, int ta, int tb, scr
         if (!rc) rc = f32_of(b, &tmpb, &xb);
         if (!rc) rc = dev_alloc((void **)&tb_f, sizeof(float) * (size_t)k * n);
         if (!rc) rc = launch_round_bf16(xb, (size_t)k * n, tb_f, s);
-        if (!rc) rc = launch_matmul_f32(ra, tb_f, 1, m, k, n, ta, tb, (*out)->d, s);
+        if (!rc) rc = launch_matmul_f32(ra, tb_f, 1, m, k, n, ta, tb, nullptr, (*out)->d, s);
         if (!rc) rc = sync();
         dev_free(ra);
         dev_free(tmpb);
@@ -698,13 +698,13 @@ int scry_hip_matmul(scry_buf a, scry_buf b, int m, int k, int n, int trans_a, in
     CHECK_BUF(b, "matmul");
     SCRY_TRY(check_mkn(a->n, b->n, m, k, n));
     SCRY_TRY(new_buf((size_t)m * n, out));
-    return launch_matmul_f32(a->d, b->d, 1, m, k, n, trans_a, trans_b, (*out)->d, ctx().stream);
+    return launch_matmul_f32(a->d, b->d, 1, m, k, n, trans_a, trans_b, nullptr, (*out)->d, ctx().stream);
 }
 
 // MathBackend::matmul_bias (mod.rs:62-86; the CUDA backend keeps the default):
 // the matmul above (bf16 operands in bf16 mode), then the f32 bias row added
-// to every output row on the device.  A bf16-only bias is widened first, as
-// the default's to_vec does.
+// to every output row on the device (in the f32 matmul's epilogue).  A
+// bf16-only bias is widened first, as the default's to_vec does.
 int scry_hip_matmul_bias(scry_buf a, scry_buf b, scry_buf bias, int m, int k, int n, int trans_a,
                          int trans_b, scry_buf *out) {
     API_LOCK;
@@ -713,11 +713,21 @@ int scry_hip_matmul_bias(scry_buf a, scry_buf b, scry_buf bias, int m, int k, in
     if (n > 0 && bias->n < (size_t)n)
         return set_error(SCRY_ERR_INVALID, "matmul_bias: bias holds %zu values, needs %d",
                          bias->n, n);
-    SCRY_TRY(scry_hip_matmul(a, b, m, k, n, trans_a, trans_b, out));
     float *tmp = nullptr;
     const float *bv = nullptr;
-    int rc = f32_of(bias, &tmp, &bv);
-    if (!rc) rc = launch_add_bias_rows((*out)->d, bv, m, n, ctx().stream);
+    int rc = SCRY_OK;
+    if (ctx().bf16) {
+        SCRY_TRY(scry_hip_matmul(a, b, m, k, n, trans_a, trans_b, out));
+        rc = f32_of(bias, &tmp, &bv);
+        if (!rc) rc = launch_add_bias_rows((*out)->d, bv, m, n, ctx().stream);
+    } else {
+        CHECK_BUF(a, "matmul");
+        CHECK_BUF(b, "matmul");
+        SCRY_TRY(check_mkn(a->n, b->n, m, k, n));
+        SCRY_TRY(new_buf((size_t)m * n, out));
+        rc = f32_of(bias, &tmp, &bv);
+        if (!rc) rc = launch_matmul_f32(a->d, b->d, 1, m, k, n, trans_a, trans_b, bv, (*out)->d, ctx().stream);
+    }
     if (tmp && !rc) rc = sync();  // the widened copy is freed below
     dev_free(tmp);
     if (rc) {
@@ -738,7 +748,7 @@ int scry_hip_matmul_strided_batched(scry_buf a, scry_buf b, int batch, int m, in
     if (a->n < (size_t)batch * m * k || b->n < (size_t)batch * k * n)
         return set_error(SCRY_ERR_INVALID, "matmul_strided_batched: operand too short");
     SCRY_TRY(new_buf((size_t)batch * m * n, out));
-    return launch_matmul_f32(a->d, b->d, batch, m, k, n, trans_a, trans_b, (*out)->d, ctx().stream);
+    return launch_matmul_f32(a->d, b->d, batch, m, k, n, trans_a, trans_b, nullptr, (*out)->d, ctx().stream);
 }
 
 int scry_hip_rmsnorm(scry_buf x, scry_buf w, int rows, int d, float eps, scry_buf *out) {

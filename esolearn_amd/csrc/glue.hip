@@ -145,29 +145,6 @@ __global__ void k_repeat_kv(const float *__restrict__ x, int n_kv, int n_q, int 
     }
 }
 
-// Generic f32 (batched) matmul, one thread per output: f64 accumulation in
-// increasing p (the reference's m > 1 fallback, cpu.rs:875-999; its m == 1
-// GEMV sums in f32 -- the difference is within f32 rounding).
-__global__ void k_matmul_f32(const float *__restrict__ a, const float *__restrict__ b, int batch,
-                             int m, int k, int n, int ta, int tb, float *__restrict__ c) {
-    const size_t total = (size_t)batch * m * n;
-    GRID_STRIDE(t, total) {
-        const int j = (int)(t % n);
-        const size_t bi = t / n;
-        const int i = (int)(bi % m);
-        const size_t bt = bi / m;
-        const float *A = a + bt * (size_t)m * k;
-        const float *B = b + bt * (size_t)k * n;
-        double acc = 0.0;
-        for (int p = 0; p < k; p++) {
-            const double av = ta ? (double)A[(size_t)p * m + i] : (double)A[(size_t)i * k + p];
-            const double bv = tb ? (double)B[(size_t)j * k + p] : (double)B[(size_t)p * n + j];
-            acc += av * bv;
-        }
-        c[t] = (float)acc;
-    }
-}
-
 // Logits of the int8 LM head for rows whose normalised input holds an
 // infinity or a NaN.  The prefill GEMMs mark such a row and give NaN for all
 // of it, while the reference's sum of f64(a) (q s) over k (cpu.rs:1128-1160)
@@ -300,15 +277,6 @@ int launch_repeat_kv(const float *x, int n_kv, int n_q, int seq, int d_head, flo
     if (total == 0) return SCRY_OK;
     hipLaunchKernelGGL(k_repeat_kv, dim3(grid1(total)), dim3(256), 0, s, x, n_kv, n_q, seq, d_head,
                        out);
-    LAUNCH_CHECK();
-}
-
-int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, int n, int ta,
-                      int tb, float *c, hipStream_t s) {
-    const size_t total = (size_t)batch * m * n;
-    if (total == 0) return SCRY_OK;
-    hipLaunchKernelGGL(k_matmul_f32, dim3(grid1(total)), dim3(256), 0, s, a, b, batch, m, k, n, ta,
-                       tb, c);
     LAUNCH_CHECK();
 }
 

@@ -280,8 +280,10 @@ int launch_gather_repeat_kv(const float *cache, int cached_len, int n_kv, int n_
                             float *out, hipStream_t s);
 int launch_repeat_kv(const float *x, int n_kv, int n_q, int seq, int d_head, float *out,
                      hipStream_t s);
-int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, int n, int ta,
-                      int tb, float *c, hipStream_t s);
+// matmul.hip: f64 accumulation, one rounding; then bias [n] (may be null) is
+// added in f32
+int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, int n, int ta, int tb,
+                      const float *bias, float *c, hipStream_t s);
 int launch_argmax(const float *x, int64_t n, int64_t *out, hipStream_t s);
 int launch_fill_f32(float *p, size_t n, float v, hipStream_t s);
 int launch_fill_u32(unsigned int *p, size_t n, unsigned int v, hipStream_t s);

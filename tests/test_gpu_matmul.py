@@ -1,0 +1,63 @@
+"""f32 matmul with f64 accumulation (matmul, matmul_bias, matmul_strided_batched;
+mod.rs:54-86, 561-591) at the edges of its kernels: 1-4 rows (row and column
+streams, their k splits and ragged widths), the 32 and 64 tiles, k tails of a
+32-value step, k splits, and every transpose.  f32 products are exact in f64,
+so a result differs from the f64 reference by its one rounding (2^-24) and the
+order of f64 additions (k 2^-53 of the sum of magnitudes, far below it)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+SHAPES = [  # batch, m, k, n
+    (1, 1, 1, 1), (2, 1, 129, 77), (32, 1, 101, 128), (1, 2, 1001, 12), (3, 3, 33, 70), (1, 4, 4100, 260),
+    (1, 1, 2048, 4100), (1, 5, 3, 7), (2, 33, 31, 65), (3, 17, 100, 129), (1, 37, 128, 37), (1, 200, 768, 50),
+    (1, 65, 2052, 68), (1, 70, 4097, 66), (12, 64, 64, 64), (1, 1030, 70, 1029),
+]
+
+
+def _check(c, a, b, extra=0.0):
+    ref = np.matmul(a.astype(np.float64), b.astype(np.float64)) + extra
+    mag = np.matmul(np.abs(a).astype(np.float64), np.abs(b).astype(np.float64)) + np.abs(extra)
+    bound = 2.0 ** -23 * np.abs(ref) + a.shape[-1] * 2.0 ** -52 * mag
+    assert (np.abs(c.astype(np.float64) - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("bt,m,k,n", SHAPES)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_matmul_f64_accumulation(hip, bt, m, k, n, ta, tb):
+    print(f"[case] {bt} x {m} x {k} x {n} ta={ta} tb={tb}", flush=True)
+    B = hip.HipBackend
+    rng = np.random.default_rng(m * k + n + bt)
+    a = rng.normal(size=(bt, m, k)).astype(F)
+    b = rng.normal(size=(bt, k, n)).astype(F)
+    A = B.from_vec(np.ascontiguousarray(a.swapaxes(1, 2) if ta else a))
+    W = B.from_vec(np.ascontiguousarray(b.swapaxes(1, 2) if tb else b))
+    c = B.matmul_strided_batched(A, W, bt, m, k, n, bool(ta), bool(tb)).to_vec().reshape(bt, m, n)
+    _check(c, a, b)
+    if bt == 1:
+        bias = rng.normal(size=n).astype(F)
+        plain = B.matmul(A, W, m, k, n, bool(ta), bool(tb)).to_vec()
+        assert np.array_equal(plain, c.ravel())
+        got = B.matmul_bias(A, W, B.from_vec(bias), m, k, n, bool(ta), bool(tb)).to_vec()
+        assert np.array_equal(got, (plain.reshape(m, n) + bias).ravel())  # the rounded product, then an f32 add
+
+
+@pytest.mark.parametrize("m", [1, 3, 40])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_matmul_nonfinite_stays_in_its_rows_and_columns(hip, m, ta, tb):
+    """Padding must not turn an infinity into a NaN elsewhere."""
+    print(f"[case] m={m} ta={ta} tb={tb}", flush=True)
+    B = hip.HipBackend
+    k, n = 37, 45
+    rng = np.random.default_rng(m)
+    a = np.abs(rng.normal(size=(m, k))).astype(F) + F(0.1)
+    b = np.abs(rng.normal(size=(k, n))).astype(F) + F(0.1)
+    a[m // 2, 5] = np.inf
+    b[7, n - 1] = np.nan
+    c = B.matmul(B.from_vec(np.ascontiguousarray(a.T if ta else a)), B.from_vec(np.ascontiguousarray(b.T if tb else b)),
+                 m, k, n, bool(ta), bool(tb)).to_vec().reshape(m, n)
+    with np.errstate(invalid="ignore"):
+        ref = (a.astype(np.float64) @ b.astype(np.float64)).astype(F)
+    assert np.array_equal(np.isnan(c), np.isnan(ref)) and np.array_equal(np.isinf(c), np.isinf(ref))

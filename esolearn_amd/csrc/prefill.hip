@@ -294,6 +294,8 @@ struct GemmP {
     const int *ae;          // row exponents
     size_t dstride;
     float *of;              // SwiGLU output as f32 rows [M][ldo] instead of the planes (k_gemm_digits)
+    int splits, kchunk;     // k_gemm_digits' smaller tiles: k splits of kchunk steps each
+    double *part;           // splits > 1: sums [split][M][N]
 };
 
 // Workgroup -> tile: workgroup b runs on XCD b % 8.  Tiles are grouped in
@@ -422,12 +424,12 @@ __device__ __forceinline__ void gemm_store(const GemmP &p, const f32x4 (&acc)[TM
 // rounding.
 __device__ __forceinline__ float silu_split(float g) { return g / (1.f + expf(-g)); }
 
-template <int TM, int TN, int NT, bool EXACT>
+template <int TM, int TN, int NT, bool EXACT, int BM_ = BM, int BN_ = BN>
 __device__ __forceinline__ void swiglu_store(const GemmP &p, const f32x4 (&acc)[TM][TN], u16 *so, int ml, int nl, int m0,
                                              int n0, int lane) {
-    constexpr int OW = BN / 2, LDO = OW + 8;  // output columns per tile; LDS row stride (u16)
+    constexpr int OW = BN_ / 2, LDO = OW + 8;  // output columns per tile; LDS row stride (u16)
     constexpr int LDF = OW + 4;               // the same in f32 (p.of: f32 rows instead of planes)
-    u16 *sh = so, *sl = so + BM * LDO;
+    u16 *sh = so, *sl = so + BM_ * LDO;
     float *sf = reinterpret_cast<float *>(so);
     const int fr = lane & 15;
 #pragma unroll
@@ -465,7 +467,7 @@ __device__ __forceinline__ void swiglu_store(const GemmP &p, const f32x4 (&acc)[
     const int oc0 = n0 >> 1, ocn = p.N >> 1;
     if (p.of) {  // f32 rows: 4 columns per 16-byte store
         constexpr int CPF = OW / 4;
-        for (int idx = threadIdx.x; idx < BM * CPF; idx += NT) {
+        for (int idx = threadIdx.x; idx < BM_ * CPF; idx += NT) {
             const int r = idx / CPF, c = idx - r * CPF;
             const int m = m0 + r, col = oc0 + c * 4;
             if (m >= p.M || col >= ocn) continue;
@@ -480,8 +482,8 @@ __device__ __forceinline__ void swiglu_store(const GemmP &p, const f32x4 (&acc)[
         return;
     }
     constexpr int CPR = OW / 8;  // 16-byte chunks per row
-    for (int idx = threadIdx.x; idx < 2 * BM * CPR; idx += NT) {
-        const int pl = idx / (BM * CPR), rem = idx - pl * (BM * CPR), r = rem / CPR, c = rem - r * CPR;
+    for (int idx = threadIdx.x; idx < 2 * BM_ * CPR; idx += NT) {
+        const int pl = idx / (BM_ * CPR), rem = idx - pl * (BM_ * CPR), r = rem / CPR, c = rem - r * CPR;
         const int m = m0 + r, col = oc0 + c * 8;
         if (m >= p.M || col >= ocn) continue;
         const u16 *src = (pl ? sl : sh) + r * LDO + c * 8;
@@ -864,44 +866,74 @@ __global__ __launch_bounds__(ring::T, 1) void k_gemm_ring(GemmP p) {
 // chunk c of row r at c ^ ((r >> 1) & 3).  Lane group g of a 16x16x64 MFMA
 // reads chunk g of its row / column for both operands, so every k pairs with
 // itself.  8 waves of 64 x 64 outputs, 120 KB of LDS, one workgroup per CU.
-namespace dring {
-constexpr int WGM = 2, WGN = 4, TM = 4, TN = 4, NW = WGM * WGN, T = 64 * NW, S = 3;
-static_assert(WGM * TM * 16 == BM && WGN * TN * 16 == BN && BK == 64, "digit ring tile");
-constexpr int A_PL = BM * BK, B_ST = BN * BK, STAGE = 3 * A_PL + B_ST;
-constexpr int A_UNITS = A_PL / 1024, B_UNITS = B_ST / 1024;  // 1 KB loads (16 rows of 64 B)
-constexpr int JA = A_UNITS / NW, JB = B_UNITS / NW, L = 3 * JA + JB;
-static_assert(A_UNITS % NW == 0 && B_UNITS % NW == 0, "digit ring units");
-constexpr size_t LDS = (size_t)S * STAGE;
-static_assert(L * (S - 2) < 64, "vmcnt range");
-static_assert(LDS >= 2 * BM * (BN / 2 + 8) * sizeof(u16) && LDS >= BM * (BN / 2 + 4) * sizeof(float),
-              "SwiGLU staging tile");
-}  // namespace dring
+// Small row counts (short prompts, the op-level matmul) leave most CUs idle
+// with that tile (512 rows x 4096 columns: 64 workgroups), so launch_gemm also
+// picks smaller tiles and splits k: a split writes its exact sums S (integers
+// below 2^53) as f64, and k_digits_finish adds them (exactly, in any order)
+// and applies the same scale, rounding and epilogue: the same bits whatever
+// the tile and the split.
+template <int BM_, int BN_, int WGM_, int WGN_, int S_>
+struct DTile {
+    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, S = S_;
+    static constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16, NW = WGM * WGN, T = 64 * NW;
+    static constexpr int A_PL = BM * BK, B_ST = BN * BK, STAGE = 3 * A_PL + B_ST;
+    static constexpr int JP = 3 * A_PL / 1024 / NW, JB = B_ST / 1024 / NW, L = JP + JB;  // 1 KB loads (16 rows of 64 B)
+    static constexpr size_t LDS = (size_t)S * STAGE;
+    static constexpr bool BIG = BM_ == 128 && BN_ == 256;  // k_gemm_ring's tile and map
+    static_assert(BK == 64 && WGM * TM * 16 == BM && WGN * TN * 16 == BN, "digit ring tile");
+    static_assert(3 * A_PL / 1024 % NW == 0 && B_ST / 1024 % NW == 0, "digit ring units");
+    static_assert(L * (S - 2) < 64, "vmcnt range");
+    static_assert(LDS >= BM * (BN / 2 + 4) * sizeof(float), "SwiGLU staging tile");
+};
+using DBig = DTile<BM, BN, 2, 4, 3>;
+static_assert(DBig::LDS >= 2 * BM * (BN / 2 + 8) * sizeof(u16), "SwiGLU plane staging tile");
 
-template <int EPI>
-__global__ __launch_bounds__(dring::T, 1) void k_gemm_digits(GemmP p) {
-    using namespace dring;
+// Workgroup -> (tile, k split) of the smaller tiles: XCD b % 8 walks a
+// contiguous run, row tiles fastest, so the row tiles of one weight panel
+// share an L2 (the super-tile map would leave XCDs without work here).
+__device__ __forceinline__ bool digit_tile(const GemmP &p, int &mb, int &nb, int &sp) {
+    const unsigned total = (unsigned)p.n_mb * p.n_nb * p.splits, per = (total + 7) / 8;
+    const unsigned w = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per || w >= total) return false;
+    mb = (int)(w % p.n_mb);
+    nb = (int)(w / p.n_mb % p.n_nb);
+    sp = (int)(w / ((unsigned)p.n_mb * p.n_nb));
+    return true;
+}
+
+// S 2^-E scale in f64, one rounding to f32
+__device__ __forceinline__ float digit_value(double S, int E, double sc) {
+    return E == DG_NONFINITE ? __builtin_nanf("") : (float)(S * ldexp(1.0, -E) * sc);
+}
+
+template <int EPI, class TL>
+__global__ __launch_bounds__(TL::T, TL::BIG ? 1 : 2) void k_gemm_digits(GemmP p) {
+    constexpr int TM = TL::TM, TN = TL::TN, NW = TL::NW, T = TL::T, S = TL::S, A_PL = TL::A_PL, STAGE = TL::STAGE;
+    constexpr int JP = TL::JP, L = TL::L, AU = A_PL / 1024;
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     extern __shared__ float4 dsm[];
     unsigned char *sm = reinterpret_cast<unsigned char *>(dsm);
-    int mb, nbk;
-    if (!gemm_tile(p, mb, nbk)) return;
-    const int m0 = mb * BM, n0 = nbk * BN;
+    int mb, nbk, sp = 0;
+    if (TL::BIG ? !gemm_tile(p, mb, nbk) : !digit_tile(p, mb, nbk, sp)) return;
+    const int m0 = mb * TL::BM, n0 = nbk * TL::BN;
+    // this split's k steps
+    const int kt0 = TL::BIG ? 0 : sp * p.kchunk, kt1 = TL::BIG ? p.nk : min(p.nk, kt0 + p.kchunk);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int wm = wave / WGN, wn = wave % WGN;
+    const int wm = wave / TL::WGN, wn = wave % TL::WGN;
     const u32x4 da = ring_desc(p.ad, 3 * p.dstride), dw = ring_desc(p.w, (size_t)p.N * p.kp);
     const unsigned sm0 = (unsigned)(uintptr_t)sm;  // LDS address (low half of the flat address)
-    // load j of this wave fills 1 KB block u = j NW + wave: j < 3 JA digit
-    // plane j / JA (16 rows of 64 B), else the weights (16 columns of 64 B)
+    // load j of this wave fills 1 KB block u = j NW + wave: digit plane u / AU
+    // (16 rows of 64 B) for j < JP, then the weights (16 columns of 64 B)
     unsigned voff[L], loff[L];
 #pragma unroll
     for (int j = 0; j < L; j++) {
-        if (j < 3 * JA) {
-            const int pl = j / JA, ua = (j % JA) * NW + wave;
+        if (j < JP) {
+            const int u = j * NW + wave, pl = u / AU, ua = u % AU;
             const int r = 16 * ua + (lane >> 2), c = (lane & 3) ^ ((r >> 1) & 3);
             voff[j] = (unsigned)(pl * p.dstride + (size_t)(m0 + r) * p.lda + c * 16);
             loff[j] = (unsigned)(pl * A_PL + ua * 1024);
         } else {
-            const int ub = (j - 3 * JA) * NW + wave;
+            const int ub = (j - JP) * NW + wave;
             const int n = 16 * ub + (lane >> 2), c = (lane & 3) ^ ((n >> 1) & 3);
             const int row = min(n0 + n, p.N - 1);  // columns past N re-read row N - 1 (never stored)
             voff[j] = (unsigned)(row * p.kp + c * 16);
@@ -910,10 +942,10 @@ __global__ __launch_bounds__(dring::T, 1) void k_gemm_digits(GemmP p) {
     }
     // step kt into ring slot; steps past the last re-read the last (in bounds, never used)
     auto issue = [&](int kt, int slot) {
-        const unsigned ko = (unsigned)(min(kt, p.nk - 1) * BK);
+        const unsigned ko = (unsigned)(min(kt, kt1 - 1) * BK);
         const unsigned base = sm0 + (unsigned)(slot * STAGE);
 #pragma unroll
-        for (int j = 0; j < L; j++) ring_load(j < 3 * JA ? da : dw, base + loff[j], voff[j], ko);
+        for (int j = 0; j < L; j++) ring_load(j < JP ? da : dw, base + loff[j], voff[j], ko);
     };
 
     i32x4 acc[3][TM][TN];
@@ -925,10 +957,10 @@ __global__ __launch_bounds__(dring::T, 1) void k_gemm_digits(GemmP p) {
             for (int j = 0; j < TN; j++) acc[d][i][j] = i32x4{0, 0, 0, 0};
     ring_wait<0>();
 #pragma unroll
-    for (int s = 0; s < S - 1; s++) issue(s, s);
+    for (int s = 0; s < S - 1; s++) issue(kt0 + s, s);
     const int fr = lane & 15, g = lane >> 4;
     int cur = 0;  // ring slot of step kt
-    for (int kt = 0; kt < p.nk; kt++) {
+    for (int kt = kt0; kt < kt1; kt++) {
         ring_wait<L * (S - 2)>();  // this wave's loads of step kt have landed
         ring_barrier();            // every wave's have; slot kt - 1 is free
         issue(kt + S - 1, cur == 0 ? S - 1 : cur - 1);
@@ -957,7 +989,25 @@ __global__ __launch_bounds__(dring::T, 1) void k_gemm_digits(GemmP p) {
         }
     }
     ring_wait<0>();  // the re-read tail steps land before the workgroup's LDS is reused or released
-    // S 2^-E scale, one rounding to f32; the store epilogues then run at unit scale
+    auto sum_of = [&](int tm, int tn, int r) {
+        return (double)acc[2][tm][tn][r] * 65536.0 + (double)acc[1][tm][tn][r] * 256.0 + (double)acc[0][tm][tn][r];
+    };
+    if (!TL::BIG && p.splits > 1) {
+        double *part = p.part + (size_t)sp * p.M * p.N;
+#pragma unroll
+        for (int tn = 0; tn < TN; tn++) {
+            const int n = n0 + wn * TN * 16 + tn * 16 + fr;
+#pragma unroll
+            for (int tm = 0; tm < TM; tm++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int m = m0 + wm * TM * 16 + tm * 16 + (g << 2) + r;
+                    if (m < p.M && n < p.N) part[(size_t)m * p.N + n] = sum_of(tm, tn, r);
+                }
+        }
+        return;
+    }
+    // the scale and the rounding here; the store epilogues then run at unit scale
     int er[TM][4];
 #pragma unroll
     for (int tm = 0; tm < TM; tm++)
@@ -974,21 +1024,55 @@ __global__ __launch_bounds__(dring::T, 1) void k_gemm_digits(GemmP p) {
 #pragma unroll
         for (int tm = 0; tm < TM; tm++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const double S = (double)acc[2][tm][tn][r] * 65536.0 + (double)acc[1][tm][tn][r] * 256.0 +
-                                 (double)acc[0][tm][tn][r];
-                const int E = er[tm][r];
-                v[tm][tn][r] = E == DG_NONFINITE ? __builtin_nanf("") : (float)(S * ldexp(1.0, -E) * sc);
-            }
+            for (int r = 0; r < 4; r++) v[tm][tn][r] = digit_value(sum_of(tm, tn, r), er[tm][r], sc);
     }
     GemmP q = p;
     q.scale = q.scale2 = 1.f;
     if (EPI == GE_SWIGLU) {
         __syncthreads();  // every wave's tail loads have landed
-        swiglu_store<TM, TN, T, false>(q, v, reinterpret_cast<u16 *>(sm), wm * TM * 16, wn * TN * 16, m0, n0, lane);
-        if (!p.of && wave == 0 && nbk == p.n_nb - 1) swiglu_pad(p, m0, lane);
+        swiglu_store<TM, TN, T, false, TL::BM, TL::BN>(q, v, reinterpret_cast<u16 *>(sm), wm * TM * 16, wn * TN * 16, m0,
+                                                       n0, lane);
+        if (TL::BIG && !p.of && wave == 0 && nbk == p.n_nb - 1) swiglu_pad(p, m0, lane);
     } else {
         gemm_store<EPI, TM, TN>(q, v, m0 + wm * TM * 16, n0 + wn * TN * 16, lane, 1.f, 1.f);
+    }
+}
+
+// The k splits' sums, added in split order; then gemm_store's (swiglu_store's,
+// f32 rows) value and epilogue.  One thread per row and 4 columns (one SwiGLU
+// group: gate, gate, up, up).  Bound by reading the partials once.
+template <int EPI>
+__global__ __launch_bounds__(256) void k_digits_finish(GemmP p) {
+    const int nq = (p.N + 3) >> 2;
+    const size_t mn = (size_t)p.M * p.N, total = (size_t)p.M * nq;
+    const bool vec = p.N % 2 == 0;  // 16-byte pairs of doubles
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (size_t)gridDim.x * 256) {
+        const int m = (int)(t / nq), n = (int)(t % nq) * 4, w = min(4, p.N - n);
+        const double *src = p.part + (size_t)m * p.N + n;
+        double S[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int sp = 0; sp < p.splits; sp++) {
+            const double *q = src + (size_t)sp * mn;
+            if (vec) {
+                const double2 a = *(const double2 *)q, b = w > 2 ? *(const double2 *)(q + 2) : make_double2(0.0, 0.0);
+                S[0] += a.x, S[1] += a.y, S[2] += b.x, S[3] += b.y;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) S[e] += e < w ? q[e] : 0.0;
+            }
+        }
+        const int E = p.ae[m];
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            v[e] = digit_value(S[e], E, EPI == GE_SWIGLU && e >= 2 ? (double)p.scale2 : (double)p.scale);
+        if (EPI == GE_SWIGLU) {
+            *(float2 *)(p.of + (size_t)m * p.ldo + (n >> 1)) =
+                make_float2(silu_split(v[0]) * v[2], silu_split(v[1]) * v[3]);
+        } else {
+            float *c = p.c + (size_t)m * p.ldc + n;
+            for (int e = 0; e < w; e++)
+                c[e] = EPI == GE_RESID ? c[e] + v[e] : EPI == GE_STORE && p.bias ? v[e] + p.bias[n + e] : v[e];
+        }
     }
 }
 
@@ -1559,17 +1643,81 @@ int gemm_t(const GemmP &p, hipStream_t s) {
     PF_LAUNCH_CHECK();
 }
 
-template <int EPI>
-int gemm_digits_t(const GemmP &p, hipStream_t s) {
+template <int EPI, class TL>
+int digits_launch(const GemmP &p, int grid, hipStream_t s) {
     static bool attr = false;
     if (!attr) {
-        SCRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gemm_digits<EPI>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)dring::LDS));
+        SCRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gemm_digits<EPI, TL>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)TL::LDS));
         attr = true;
     }
-    const int grid = (p.n_super + 7) / 8 * 8 * 32;
-    hipLaunchKernelGGL((k_gemm_digits<EPI>), dim3(grid), dim3(dring::T), dring::LDS, s, p);
+    hipLaunchKernelGGL((k_gemm_digits<EPI, TL>), dim3(grid), dim3(TL::T), TL::LDS, s, p);
     PF_LAUNCH_CHECK();
+}
+
+template <int EPI, class TL>
+int digits_small(GemmP p, int splits, hipStream_t s) {
+    p.n_mb = (p.M + TL::BM - 1) / TL::BM;
+    p.n_nb = (p.N + TL::BN - 1) / TL::BN;
+    p.kchunk = (p.nk + splits - 1) / splits;
+    p.splits = (p.nk + p.kchunk - 1) / p.kchunk;
+    if (p.splits > 1) {
+        void *ws = nullptr;
+        SCRY_TRY(ctx_workspace(sizeof(double) * (size_t)p.splits * p.M * p.N, &ws));
+        p.part = (double *)ws;
+    }
+    SCRY_TRY((digits_launch<EPI, TL>(p, (p.n_mb * p.n_nb * p.splits + 7) / 8 * 8, s)));
+    if (p.splits > 1) {
+        const size_t g = ((size_t)p.M * ((p.N + 3) / 4) + 255) / 256;
+        hipLaunchKernelGGL(k_digits_finish<EPI>, dim3((unsigned)std::min<size_t>(g, 65536)), dim3(256), 0, s, p);
+        PF_LAUNCH_CHECK();
+    }
+    return SCRY_OK;
+}
+
+// Tile and k splits for M rows.  The time of a choice: k steps of a split times
+// the workgroups each CU runs one after another or together (workgroups / 256)
+// times the measured time of one workgroup's step (us, from 17-1024 rows at
+// k 768-11008, n 768-22016: alone on a CU / sharing it), plus the f64 partial
+// sums' round trip.  Measured, old tile -> this choice: 512 x 11008 x 4096
+// (rows, k, n) 193 -> 91 us, 512 x 4096 x 4096 81 -> 43, 130 x 4096 x 14336
+// 80 -> 57, 64 x 11008 x 4096 180 -> 29, 200 x 768 x 2304 26 -> 11; from about
+// 224 tiles of 128 x 256 on the large tile stays the fastest (512 x 4096 x
+// 14336: 89 us against 113, 1024 x 4096 x 22016: 245 against 324).
+struct DigitPick {
+    int tile, splits;
+};
+DigitPick pick_digits(int M, int N, int nk, bool small_ok) {
+    struct {
+        int bm, bn;
+        double alone, shared;
+    } const tl[] = {{128, 256, 1.25, 1.25}, {128, 128, 0.80, 0.80}, {64, 128, 0.52, 0.50}, {64, 64, 0.38, 0.345}, {32, 128, 0.376, 0.34}};
+    DigitPick best{0, 1};
+    double bt = 1e30;
+    for (int i = 0; i < (small_ok ? 5 : 1); i++) {
+        const double tiles = (double)((M + tl[i].bm - 1) / tl[i].bm) * ((N + tl[i].bn - 1) / tl[i].bn);
+        for (int sp = 1; sp <= (i ? 16 : 1); sp *= 2) {
+            if (sp > 1 && (nk < 4 * sp || (double)sp * M * N > 33554432.0)) break;  // at most 256 MB of partials
+            const double n = std::ceil(tiles * sp / 256.0);
+            double t = (nk + sp - 1) / sp * n * (n > 1 ? tl[i].shared : tl[i].alone);
+            if (sp > 1) t += 4.0 + (double)sp * M * N * 16.0 / 5.0e6;
+            if (t < bt) bt = t, best = {i, sp};
+        }
+    }
+    return best;
+}
+
+template <int EPI>
+int gemm_digits_t(const GemmP &p, hipStream_t s) {
+    // the smaller tiles write SwiGLU as f32 rows only
+    const DigitPick d = pick_digits(p.M, p.N, p.nk, EPI != GE_SWIGLU || p.of);
+    switch (d.tile) {
+        case 1: return digits_small<EPI, DTile<128, 128, 2, 4, 3>>(p, d.splits, s);
+        case 2: return digits_small<EPI, DTile<64, 128, 2, 2, 3>>(p, d.splits, s);
+        case 3: return digits_small<EPI, DTile<64, 64, 2, 2, 4>>(p, d.splits, s);
+        case 4: return digits_small<EPI, DTile<32, 128, 1, 2, 4>>(p, d.splits, s);
+    }
+    return digits_launch<EPI, DBig>(p, (p.n_super + 7) / 8 * 8 * 32, s);
 }
 
 template <int EPI, bool WBF>

@@ -1,0 +1,57 @@
+"""The digit GEMM's tiles and k splits (matmul_i8_f32 above 16 rows, the int8
+model's prefill): small integer activations have exact digit planes, so every
+tile and split must give the exact integer sums; and a model whose prefill
+GEMMs split k against its token-by-token decode."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+F = np.float32
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (17, 64, 5), (33, 100, 131), (32, 2048, 128), (37, 4096, 260), (64, 768, 768), (65, 3072, 770),
+    (130, 4096, 1030), (200, 768, 2304), (129, 8192, 4096), (300, 1024, 4097), (512, 2048, 2050)])
+def test_exact_sums(hip, m, k, n):
+    print(f"[case] {m} x {k} x {n}", flush=True)
+    B = hip.HipBackend
+    rng = np.random.default_rng(m + k + n)
+    a = rng.integers(-8, 9, (m, k)).astype(F)
+    q = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    bias = rng.integers(-100, 100, n).astype(F)
+    ref = a.astype(np.float64) @ q.astype(np.float64)  # below 2^24: exact in f32
+    A, W = B.from_vec(a), B.i8_from_vec(q)
+    assert np.array_equal(B.matmul_i8_f32(A, W, 1.0, m, k, n).to_vec().reshape(m, n), ref)
+    assert np.array_equal(B.matmul_i8_f32_bias(A, W, 1.0, B.from_vec(bias), m, k, n).to_vec().reshape(m, n), ref + bias)
+
+
+def test_nonfinite_row_only(hip):
+    """A row holding an infinity is NaN as a whole, its neighbours are untouched (k splits included)."""
+    B = hip.HipBackend
+    m, k, n = 40, 4096, 256
+    rng = np.random.default_rng(3)
+    a = rng.integers(-8, 9, (m, k)).astype(F)
+    q = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    ref = a.astype(np.float64) @ q.astype(np.float64)
+    a[7, 100] = np.inf
+    c = B.matmul_i8_f32(B.from_vec(a), B.i8_from_vec(q), 1.0, m, k, n).to_vec().reshape(m, n)
+    assert np.isnan(c[7]).all()
+    keep = np.arange(m) != 7
+    assert np.array_equal(c[keep], ref[keep])
+
+
+@pytest.mark.parametrize("seq", [18, 70, 130])
+def test_prefill_with_split_k_matches_decode(hip, seq):
+    """hidden 2048, ffn 4100: the residual and SwiGLU epilogues after k splits
+    (ffn not a multiple of 8), logits within 1e-3 of the decode path's."""
+    print(f"[case] seq={seq}", flush=True)
+    cfg = hip.LlamaConfig(vocab_size=96, hidden_size=2048, intermediate_size=4100, n_layers=1, n_heads=16,
+                          n_kv_heads=4, max_seq_len=256, rope_theta=10000.0, tie_word_embeddings=False)
+    m = hip.LlamaModel.new_random(cfg, 3, init_on_device=True)
+    toks = np.random.default_rng(seq).integers(0, 96, seq)
+    cp, cd = m.new_llama_kv_cache(seq), m.new_llama_kv_cache(seq)
+    last = m.prefill([cp], toks[None, :])[0]
+    for p, t in enumerate(toks):
+        ref, _ = m.forward_with_llama_cache(int(t), p, cd)
+    assert np.abs(last - ref).max() <= 1e-3 * np.abs(ref).max()
+    m.free()

@@ -45,6 +45,11 @@ int dev_alloc(void **p, size_t bytes) {
     *p = nullptr;
     if (bytes == 0) bytes = 16;
     hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {  // give the op storage cache back and try once more
+        (void)hipGetLastError();
+        pool_trim();
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         *p = nullptr;
@@ -90,7 +95,7 @@ int new_buf(size_t n, scry_buf *out) {
     if (!out) return set_error(SCRY_ERR_INVALID, "null output handle");
     auto *b = new (std::nothrow) scry_buf_s;
     if (!b) return set_error(SCRY_ERR_OOM, "host allocation failed");
-    int rc = dev_alloc((void **)&b->d, n * sizeof(float));
+    int rc = pool_alloc((void **)&b->d, n * sizeof(float));
     if (rc) {
         delete b;
         return rc;
@@ -102,17 +107,17 @@ int new_buf(size_t n, scry_buf *out) {
 
 void del_buf(scry_buf b) {
     if (!b) return;
-    dev_free(b->d);
-    dev_free(b->bf);
-    dev_free(b->pk);
+    pool_free(b->d);
+    pool_free(b->bf);
+    pool_free(b->pk);
     delete b;
 }
 
 // the f32 data changed in place: drop the bf16 copies made from it
 void bf16_stale(scry_buf b) {
     if (!b->d) return;
-    dev_free(b->bf);
-    dev_free(b->pk);
+    pool_free(b->bf);
+    pool_free(b->pk);
     b->bf = nullptr;
     b->pk = nullptr;
     b->pk_tb = -1;
@@ -139,11 +144,11 @@ int sync() {
 // [k, n]; tb: stored [n][k]), built once per (k, n, tb)
 int bf16_rows(scry_buf b, int k, int n, int tb, const unsigned short **rows, int *kp) {
     if (!(b->pk && b->pk_k == k && b->pk_n == n && b->pk_tb == tb)) {
-        dev_free(b->pk);
+        pool_free(b->pk);
         b->pk = nullptr;
         b->pk_tb = -1;
         const int p = bf16_row_pad(k);
-        SCRY_TRY(dev_alloc((void **)&b->pk, sizeof(unsigned short) * (size_t)n * p));
+        SCRY_TRY(pool_alloc((void **)&b->pk, sizeof(unsigned short) * (size_t)n * p));
         SCRY_TRY(launch_pack_rows_bf16(b->d ? nullptr : b->bf, b->d, k, n, tb, b->pk, p, ctx().stream));
         b->pk_k = k;
         b->pk_n = n;
@@ -161,7 +166,7 @@ int f32_of(scry_buf a, float **tmp, const float **x) {
         *x = a->d;
         return SCRY_OK;
     }
-    SCRY_TRY(dev_alloc((void **)tmp, sizeof(float) * (a->n ? a->n : 1)));
+    SCRY_TRY(pool_alloc((void **)tmp, sizeof(float) * (a->n ? a->n : 1)));
     SCRY_TRY(launch_widen_bf16(a->bf, a->n, *tmp, ctx().stream));
     *x = *tmp;
     return SCRY_OK;
@@ -187,8 +192,7 @@ int matmul_bf16(scry_buf a, scry_buf b, int m, int k, int n, int ta, int tb, scr
             rc = launch_gemv_bf16(rows, kp, n, x, k, k, m, (*out)->d, n, nullptr, s);
         } else if (!rc) {
             const int mp = prefill_rows_pad(m), lda = prefill_k_pad(k);
-            rc = dev_alloc((void **)&plane, sizeof(unsigned short) * (size_t)mp * lda);
-            if (!rc) rc = launch_fill_u32((unsigned *)plane, (size_t)mp * lda / 2, 0u, s);
+            rc = pool_alloc((void **)&plane, sizeof(unsigned short) * (size_t)mp * lda);
             if (!rc) rc = launch_plane_bf16(x, k, m, k, lda, plane, lda, s);
             if (!rc) rc = launch_gemm_bf16(rows, kp, n, k, plane, lda, m, (*out)->d, n, nullptr, s);
         }
@@ -196,22 +200,20 @@ int matmul_bf16(scry_buf a, scry_buf b, int m, int k, int n, int ta, int tb, scr
         // both operands as the f32 values of their bf16 roundings
         float *ra = nullptr;
         rc = f32_of(a, &tmp, &x);
-        if (!rc) rc = dev_alloc((void **)&ra, sizeof(float) * (size_t)m * k);
+        if (!rc) rc = pool_alloc((void **)&ra, sizeof(float) * (size_t)m * k);
         if (!rc) rc = launch_round_bf16(x, (size_t)m * k, ra, s);
         const float *xb = nullptr;
         float *tmpb = nullptr;
         if (!rc) rc = f32_of(b, &tmpb, &xb);
-        if (!rc) rc = dev_alloc((void **)&tb_f, sizeof(float) * (size_t)k * n);
+        if (!rc) rc = pool_alloc((void **)&tb_f, sizeof(float) * (size_t)k * n);
         if (!rc) rc = launch_round_bf16(xb, (size_t)k * n, tb_f, s);
         if (!rc) rc = launch_matmul_f32(ra, tb_f, 1, m, k, n, ta, tb, nullptr, (*out)->d, s);
-        if (!rc) rc = sync();
-        dev_free(ra);
-        dev_free(tmpb);
+        pool_free(ra);
+        pool_free(tmpb);
     }
-    if (!rc) rc = sync();  // temporaries are freed below
-    dev_free(tmp);
-    dev_free(tb_f);
-    dev_free(plane);
+    pool_free(tmp);
+    pool_free(tb_f);
+    pool_free(plane);
     if (rc) {
         del_buf(*out);
         *out = nullptr;
@@ -276,13 +278,13 @@ int qmatmul(scry_buf a, scry_i8buf bq, float scale, const float *scales32, const
         rc = launch_qgemv(EPI_STORE, g, ctx().stream);
     } else if (gemm_takes_digits(w) && k <= 16384) {
         // prefill shapes, int8 per-tensor: the rows as digit planes (per-row
-        // 24-bit fixed point), then the GEMM on the int8 matrix cores
+        // 24-bit fixed point), then the GEMM on the int8 matrix cores (plane
+        // rows past m hold whatever was there: they feed no stored output)
         const int mp = prefill_rows_pad(m), ld = prefill_k_pad(k);
         const size_t dstride = (size_t)mp * ld;
         signed char *dg = nullptr;
-        rc = dev_alloc((void **)&dg, 3 * dstride + sizeof(int) * (size_t)mp);
+        rc = pool_alloc((void **)&dg, 3 * dstride + sizeof(int) * (size_t)mp);
         int *de = reinterpret_cast<int *>(dg + 3 * dstride);
-        if (!rc) rc = launch_fill_u32((unsigned *)dg, (3 * dstride) / 4 + mp, 0u, ctx().stream);
         if (!rc) rc = launch_norm_digits(a->d, k, m, nullptr, k, 0.f, dg, dstride, de, ld, ctx().stream);
         PrefillGemm g;
         g.w = &w;
@@ -295,14 +297,12 @@ int qmatmul(scry_buf a, scry_i8buf bq, float scale, const float *scales32, const
         g.ldc = n;
         g.bias = bias;
         if (!rc) rc = launch_gemm(PF_STORE, g, ctx().stream);
-        if (!rc) rc = sync();  // the planes are freed below
-        dev_free(dg);
+        pool_free(dg);
     } else {
         // prefill shapes: the activations as bf16 planes, then the MFMA GEMM
         const int mp = prefill_rows_pad(m), ld = prefill_k_pad(k);
         unsigned short *pl = nullptr;
-        rc = dev_alloc((void **)&pl, sizeof(unsigned short) * 2 * (size_t)mp * ld);
-        if (!rc) rc = launch_fill_u32((unsigned *)pl, (size_t)mp * ld, 0u, ctx().stream);  // 2 planes of u16
+        rc = pool_alloc((void **)&pl, sizeof(unsigned short) * 2 * (size_t)mp * ld);
         if (!rc) rc = launch_split(a->d, k, m, k, pl, pl + (size_t)mp * ld, ld, ctx().stream);
         PrefillGemm g;
         g.w = &w;
@@ -314,8 +314,7 @@ int qmatmul(scry_buf a, scry_i8buf bq, float scale, const float *scales32, const
         g.ldc = n;
         g.bias = bias;
         if (!rc) rc = launch_gemm(PF_STORE, g, ctx().stream);
-        if (!rc) rc = sync();  // the planes are freed below
-        dev_free(pl);
+        pool_free(pl);
     }
     if (rc) {
         del_buf(o);
@@ -377,6 +376,7 @@ int scry_hip_shutdown(void) {
     Ctx &c = ctx();
     if (!c.init) return SCRY_OK;
     (void)hipStreamSynchronize(c.stream);
+    pool_trim();
     dev_free(c.ws);
     (void)hipStreamDestroy(c.stream);
     c = Ctx{};
@@ -441,13 +441,13 @@ int scry_hip_to_vec(scry_buf b, float *host, size_t n) {
     if (!n) return SCRY_OK;
     if (!b->d) {  // cuda.rs:244-254: bf16-only storage widens to f32
         float *t = nullptr;
-        SCRY_TRY(dev_alloc((void **)&t, n * sizeof(float)));
+        SCRY_TRY(pool_alloc((void **)&t, n * sizeof(float)));
         int rc = launch_widen_bf16(b->bf, n, t, ctx().stream);
         hipError_t e = hipSuccess;
         if (!rc) e = hipMemcpyAsync(host, t, n * sizeof(float), hipMemcpyDeviceToHost, ctx().stream);
         if (!rc && e != hipSuccess) rc = hip_fail(e, "to_vec copy", __FILE__, __LINE__);
         if (!rc) rc = sync();
-        dev_free(t);
+        pool_free(t);
         return rc;
     }
     SCRY_HIP(hipMemcpyAsync(host, b->d, n * sizeof(float), hipMemcpyDeviceToHost, ctx().stream));
@@ -482,7 +482,7 @@ int scry_hip_from_vec_with_bf16(const float *host, const uint16_t *bf16, size_t 
     auto *b = new (std::nothrow) scry_buf_s;
     if (!b) return set_error(SCRY_ERR_OOM, "host allocation failed");
     b->n = n;
-    int rc = dev_alloc((void **)&b->bf, sizeof(uint16_t) * (n ? n : 1));
+    int rc = pool_alloc((void **)&b->bf, sizeof(uint16_t) * (n ? n : 1));
     if (!rc && n) {
         hipError_t e = hipMemcpyAsync(b->bf, bf16, sizeof(uint16_t) * n, hipMemcpyHostToDevice, ctx().stream);
         if (e != hipSuccess) rc = hip_fail(e, "from_vec_with_bf16 upload", __FILE__, __LINE__);
@@ -505,7 +505,7 @@ int scry_hip_clone_storage(scry_buf src, scry_buf *out) {
         auto *b = new (std::nothrow) scry_buf_s;
         if (!b) return set_error(SCRY_ERR_OOM, "host allocation failed");
         b->n = src->n;
-        int rc = dev_alloc((void **)&b->bf, sizeof(uint16_t) * (src->n ? src->n : 1));
+        int rc = pool_alloc((void **)&b->bf, sizeof(uint16_t) * (src->n ? src->n : 1));
         if (!rc && src->n) {
             hipError_t e = hipMemcpyAsync(b->bf, src->bf, sizeof(uint16_t) * src->n, hipMemcpyDeviceToDevice,
                                           ctx().stream);
@@ -533,7 +533,6 @@ int scry_hip_buf_len(scry_buf b, size_t *n) {
 
 int scry_hip_free(scry_buf b) {
     API_LOCK;
-    if (b && ctx().init) (void)hipStreamSynchronize(ctx().stream);
     del_buf(b);
     return SCRY_OK;
 }
@@ -600,8 +599,8 @@ int scry_hip_quantize_symmetric(scry_buf w, scry_i8buf *q_out, float *scale_out)
     unsigned int *bits = nullptr;
     float *dscale = nullptr;
     int rc = dev_alloc((void **)&q->d, w->n);
-    if (!rc) rc = dev_alloc((void **)&bits, 16);
-    if (!rc) rc = dev_alloc((void **)&dscale, 16);
+    if (!rc) rc = pool_alloc((void **)&bits, 16);
+    if (!rc) rc = pool_alloc((void **)&dscale, 16);
     if (!rc) rc = launch_absmax(w->d, w->n, bits, ctx().stream);
     if (!rc) rc = launch_quantize_plain(w->d, w->n, bits, q->d, dscale, ctx().stream);
     float s = 0.f;
@@ -610,8 +609,8 @@ int scry_hip_quantize_symmetric(scry_buf w, scry_i8buf *q_out, float *scale_out)
         if (e == hipSuccess) e = hipStreamSynchronize(ctx().stream);
         if (e != hipSuccess) rc = hip_fail(e, "quantize scale readback", __FILE__, __LINE__);
     }
-    dev_free(bits);
-    dev_free(dscale);
+    pool_free(bits);
+    pool_free(dscale);
     if (rc) {
         dev_free(q->d);
         delete q;
@@ -728,8 +727,7 @@ int scry_hip_matmul_bias(scry_buf a, scry_buf b, scry_buf bias, int m, int k, in
         rc = f32_of(bias, &tmp, &bv);
         if (!rc) rc = launch_matmul_f32(a->d, b->d, 1, m, k, n, trans_a, trans_b, bv, (*out)->d, ctx().stream);
     }
-    if (tmp && !rc) rc = sync();  // the widened copy is freed below
-    dev_free(tmp);
+    pool_free(tmp);
     if (rc) {
         del_buf(*out);
         *out = nullptr;
@@ -839,7 +837,7 @@ int scry_hip_embedding(scry_buf weight, const int64_t *ids, int n_ids, int vocab
             return set_error(SCRY_ERR_RANGE, "embedding index out of range: %lld >= vocab %d",
                              (long long)ids[i], vocab);
     int64_t *d_ids = nullptr;
-    SCRY_TRY(dev_alloc((void **)&d_ids, sizeof(int64_t) * (size_t)(n_ids ? n_ids : 1)));
+    SCRY_TRY(pool_alloc((void **)&d_ids, sizeof(int64_t) * (size_t)(n_ids ? n_ids : 1)));
     int rc = new_buf((size_t)n_ids * dim, out);
     if (!rc && n_ids) {
         hipError_t e = hipMemcpyAsync(d_ids, ids, sizeof(int64_t) * n_ids, hipMemcpyHostToDevice,
@@ -850,7 +848,7 @@ int scry_hip_embedding(scry_buf weight, const int64_t *ids, int n_ids, int vocab
                            : launch_embed_bf16((*out)->d, weight->bf, d_ids, n_ids, dim, ctx().stream);  // cuda.rs:480-503
         if (!rc) rc = sync();
     }
-    dev_free(d_ids);
+    pool_free(d_ids);
     return rc;
 }
 
@@ -900,14 +898,14 @@ int scry_hip_argmax(scry_buf logits, int64_t *out) {
     CHECK_BUF(logits, "argmax");
     if (!out) return set_error(SCRY_ERR_INVALID, "argmax: null output");
     int64_t *d = nullptr;
-    SCRY_TRY(dev_alloc((void **)&d, sizeof(int64_t)));
+    SCRY_TRY(pool_alloc((void **)&d, sizeof(int64_t)));
     int rc = launch_argmax(logits->d, (int64_t)logits->n, d, ctx().stream);
     if (!rc) {
         hipError_t e = hipMemcpyAsync(out, d, sizeof(int64_t), hipMemcpyDeviceToHost, ctx().stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx().stream);
         if (e != hipSuccess) rc = hip_fail(e, "argmax readback", __FILE__, __LINE__);
     }
-    dev_free(d);
+    pool_free(d);
     return rc;
 }
 
@@ -949,7 +947,7 @@ int scry_hip_sample_token(scry_buf logits, const scry_sampling_config *cfg, uint
     const bool prep = sample_uses_prep(*cfg, (int)V);
     const size_t pb = prep ? sample_prep_bytes((int)V) : 0;
     char *blk = nullptr;
-    SCRY_TRY(dev_alloc((void **)&blk, 64 + sizeof(double) * V + pb));
+    SCRY_TRY(pool_alloc((void **)&blk, 64 + sizeof(double) * V + pb));
     DevState *st = (DevState *)blk;
     int64_t *toks = (int64_t *)(blk + 16);
     unsigned long long *rng = (unsigned long long *)(blk + 32);
@@ -970,7 +968,7 @@ int scry_hip_sample_token(scry_buf logits, const scry_sampling_config *cfg, uint
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) rc = hip_fail(e, "sample_token readback", __FILE__, __LINE__);
     }
-    dev_free(blk);
+    pool_free(blk);
     if (rc) return rc;
     *out = h.toks[1];
     *rng_state = h.rng;
@@ -1093,7 +1091,7 @@ int scry_hip_sum(scry_buf x, float *out) {
     CHECK_BUF(x, "sum");
     if (!out) return set_error(SCRY_ERR_INVALID, "sum: null output");
     char *blk = nullptr;
-    SCRY_TRY(dev_alloc((void **)&blk, 16 + sizeof(double) * (size_t)sum_partials(x->n)));
+    SCRY_TRY(pool_alloc((void **)&blk, 16 + sizeof(double) * (size_t)sum_partials(x->n)));
     float *d_out = (float *)blk;
     int rc = launch_sum(x->d, x->n, (double *)(blk + 16), d_out, ctx().stream);
     if (!rc) {
@@ -1101,7 +1099,7 @@ int scry_hip_sum(scry_buf x, float *out) {
         if (e == hipSuccess) e = hipStreamSynchronize(ctx().stream);
         if (e != hipSuccess) rc = hip_fail(e, "sum readback", __FILE__, __LINE__);
     }
-    dev_free(blk);
+    pool_free(blk);
     return rc;
 }
 
@@ -1148,7 +1146,7 @@ int scry_hip_rope(scry_buf x, size_t rows, int last_dim, int pos, int head_dim, 
         cs[i] = make_float2((float)std::cos(ang), (float)std::sin(ang));
     }
     float2 *d_cs = nullptr;
-    SCRY_TRY(dev_alloc((void **)&d_cs, sizeof(float2) * cs.size()));
+    SCRY_TRY(pool_alloc((void **)&d_cs, sizeof(float2) * cs.size()));
     int rc = new_buf(x->n, out);
     if (!rc) {
         hipError_t e = hipMemcpyAsync(d_cs, cs.data(), sizeof(float2) * cs.size(), hipMemcpyHostToDevice,
@@ -1157,7 +1155,7 @@ int scry_hip_rope(scry_buf x, size_t rows, int last_dim, int pos, int head_dim, 
         if (!rc) rc = launch_rope_row(x->d, rows, last_dim, head_dim, d_cs, (*out)->d, ctx().stream);
         if (!rc) rc = sync();  // the table is freed below
     }
-    dev_free(d_cs);
+    pool_free(d_cs);
     return rc;
 }
 

@@ -34,6 +34,11 @@ int set_error(int code, const char *fmt, ...);
 int hip_fail(hipError_t e, const char *expr, const char *file, int line);
 int dev_alloc(void **p, size_t bytes);
 void dev_free(void *p);
+// pool.hip: device blocks for op storage and op temporaries, used on the
+// context's stream only; freed blocks are reused in stream order
+int pool_alloc(void **p, size_t bytes);
+void pool_free(void *p);
+void pool_trim();
 
 #define SCRY_HIP(expr)                                                          \
     do {                                                                        \

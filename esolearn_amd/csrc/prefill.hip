@@ -294,8 +294,9 @@ struct GemmP {
     const int *ae;          // row exponents
     size_t dstride;
     float *of;              // SwiGLU output as f32 rows [M][ldo] instead of the planes (k_gemm_digits)
-    int splits, kchunk;     // k_gemm_digits' smaller tiles: k splits of kchunk steps each
+    int splits, kchunk;     // the smaller tiles: k splits of kchunk steps each
     double *part;           // splits > 1: sums [split][M][N]
+    float *partf;           // the same for k_gemm_ring
 };
 
 // Workgroup -> tile: workgroup b runs on XCD b % 8.  Tiles are grouped in
@@ -497,10 +498,11 @@ __device__ __forceinline__ void swiglu_store(const GemmP &p, const f32x4 (&acc)[
 }
 
 // zero the plane columns past the SwiGLU output (k padding of the next GEMM),
-// rows [m0, m0 + BM); one wave of the last column tile
+// rows [m0, m0 + BM_); one wave of the last column tile
+template <int BM_>
 __device__ __forceinline__ void swiglu_pad(const GemmP &p, int m0, int lane) {
     const int c0 = p.N >> 1;
-    for (int idx = lane; idx < BM * (p.opad - c0); idx += 64) {
+    for (int idx = lane; idx < BM_ * (p.opad - c0); idx += 64) {
         const int m = m0 + idx / (p.opad - c0), col = c0 + idx % (p.opad - c0);
         p.ohi[(size_t)m * p.ldo + col] = 0;
         p.olo[(size_t)m * p.ldo + col] = 0;
@@ -650,10 +652,10 @@ __global__ __launch_bounds__(G_THREADS, B32 ? 1 : 2) void k_gemm(GemmP p) {
     // ---- epilogue: D[4 (l / 16) + r][l % 16] of each tile
     if (EPI == GE_SWIGLU && !B32) {  // (the last k step ended with a barrier: LDS is free)
         swiglu_store<4, 8, G_THREADS, WBF>(p, acc, sa, wm * 64, wn * 128, m0, n0, lane);
-        if (wave == 0 && nbk == p.n_nb - 1) swiglu_pad(p, m0, lane);
+        if (wave == 0 && nbk == p.n_nb - 1) swiglu_pad<BM>(p, m0, lane);
     } else {
         gemm_store<EPI, 4, 8>(p, acc, m0 + wm * 64, n0 + wn * 128, lane, B32 ? 1.f : p.scale, B32 ? 1.f : p.scale2);
-        if (EPI == GE_SWIGLU && wave == 0 && nbk == p.n_nb - 1) swiglu_pad(p, m0, lane);
+        if (EPI == GE_SWIGLU && wave == 0 && nbk == p.n_nb - 1) swiglu_pad<BM>(p, m0, lane);
     }
 }
 
@@ -680,23 +682,29 @@ __global__ __launch_bounds__(G_THREADS, B32 ? 1 : 2) void k_gemm(GemmP p) {
 // c ^ ((n >> 1) & 3).  MFMA k order within a step: lane group g of the
 // 16x16x32 MFMA holds k = 16 g + 8 h + e for k half h, e < 8, which makes
 // the weight operand of both halves one 16-byte read per lane.
-namespace ring {
-constexpr int WGM = 2, WGN = 4, TM = 4, TN = 4, NW = WGM * WGN, T = 64 * NW, S = 3;
-static_assert(WGM * TM * 16 == BM && WGN * TN * 16 == BN && BK == 64, "ring tile");
-// WBF: bf16 weight rows (128 B per column and step, read as they are) and
-// one activation plane (the bf16 model); else int8 weights and hi, lo planes
-template <bool WBF>
-struct Lay {
+// WBF: bf16 weight rows (128 B per column and step, read as they are) and one
+// activation plane (the bf16 model); else int8 weights and hi, lo planes.
+// The bf16 model's short prompts and the op-level bf16 matmul also take
+// smaller tiles and k splits (pick_ring): with 128 x 256, 37 rows x 4096
+// columns are 16 workgroups.  Without splits a tile changes no bit (the k
+// order is the same); a split's f32 sums are added in split order.
+template <bool WBF, int BM_, int BN_, int WGM_, int WGN_, int S_>
+struct RTile {
+    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, S = S_;
+    static constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16, NW = WGM * WGN, T = 64 * NW;
     static constexpr int NPL = WBF ? 1 : 2, WB = WBF ? 2 : 1;  // activation planes; bytes per weight
     static constexpr int A_PL = BM * BK * 2, B_ST = BN * BK * WB, STAGE = NPL * A_PL + B_ST;
     static constexpr int JA = A_PL / 1024 / NW, JB = B_ST / 1024 / NW;  // 1 KB loads per wave and step
     static constexpr int L = NPL * JA + JB;
-    static_assert((A_PL / 1024) % NW == 0 && (B_ST / 1024) % NW == 0, "ring units");
     static constexpr size_t LDS = (size_t)S * STAGE;
+    static constexpr bool BIG = BM_ == 128 && BN_ == 256;  // the super-tile map, no k splits
+    static_assert(WGM * TM * 16 == BM && WGN * TN * 16 == BN && BK == 64, "ring tile");
+    static_assert((A_PL / 1024) % NW == 0 && (B_ST / 1024) % NW == 0, "ring units");
     static_assert(L * (S - 2) < 64, "vmcnt range");
     static_assert(LDS >= 2 * BM * (BN / 2 + 8) * sizeof(u16), "SwiGLU staging tile");
 };
-}  // namespace ring
+template <bool WBF>
+using RBig = RTile<WBF, BM, BN, 2, 4, 3>;
 
 // buffer descriptor words (base, stride 0, num_records, raw-buffer flags),
 // wave-uniform
@@ -733,19 +741,33 @@ __device__ __forceinline__ void ring_wait() { asm volatile("s_waitcnt vmcnt(%0)"
 // ring's loads); LDS reads and writes of this wave complete first
 __device__ __forceinline__ void ring_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int EPI, bool WBF>
-__global__ __launch_bounds__(ring::T, 1) void k_gemm_ring(GemmP p) {
-    using namespace ring;
-    using C = Lay<WBF>;
-    constexpr int A_PL = C::A_PL, STAGE = C::STAGE, JA = C::JA, L = C::L, NPL = C::NPL, WB = C::WB;
+// Workgroup -> (tile, k split) of the smaller tiles: XCD b % 8 walks a
+// contiguous run, row tiles fastest, so the row tiles of one weight panel
+// share an L2 (the super-tile map would leave XCDs without work here).
+__device__ __forceinline__ bool small_tile(const GemmP &p, int &mb, int &nb, int &sp) {
+    const unsigned total = (unsigned)p.n_mb * p.n_nb * p.splits, per = (total + 7) / 8;
+    const unsigned w = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per || w >= total) return false;
+    mb = (int)(w % p.n_mb);
+    nb = (int)(w / p.n_mb % p.n_nb);
+    sp = (int)(w / ((unsigned)p.n_mb * p.n_nb));
+    return true;
+}
+
+template <int EPI, bool WBF, class C>
+__global__ __launch_bounds__(C::T, C::BIG ? 1 : 2) void k_gemm_ring(GemmP p) {
+    constexpr int A_PL = C::A_PL, STAGE = C::STAGE, JA = C::JA, L = C::L, NPL = C::NPL, WB = C::WB, S = C::S;
+    constexpr int TM = C::TM, TN = C::TN, NW = C::NW, T = C::T, WGN = C::WGN;
     extern __shared__ float4 rsm[];
     unsigned char *sm = reinterpret_cast<unsigned char *>(rsm);
-    int mb, nbk;
-    if (!gemm_tile(p, mb, nbk)) return;
-    const int m0 = mb * BM, n0 = nbk * BN;
+    int mb, nbk, sp = 0;
+    if (C::BIG ? !gemm_tile(p, mb, nbk) : !small_tile(p, mb, nbk, sp)) return;
+    const int m0 = mb * C::BM, n0 = nbk * C::BN;
+    // this split's k steps
+    const int kt0 = C::BIG ? 0 : sp * p.kchunk, kt1 = C::BIG ? p.nk : min(p.nk, kt0 + p.kchunk);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    const size_t a_bytes = (size_t)p.n_mb * BM * p.lda * 2;
+    const size_t a_bytes = (size_t)p.n_mb * C::BM * p.lda * 2;
     const u32x4 dh = ring_desc(p.ahi, a_bytes), dl = ring_desc(WBF ? p.ahi : p.alo, a_bytes);
     const u32x4 dw = ring_desc(p.w, (size_t)p.N * p.kp * WB);
     const unsigned sm0 = (unsigned)(uintptr_t)sm;  // LDS address (low half of the flat address)
@@ -776,7 +798,7 @@ __global__ __launch_bounds__(ring::T, 1) void k_gemm_ring(GemmP p) {
     }
     // step kt into ring slot; steps past the last re-read the last (in bounds, never used)
     auto issue = [&](int kt, int slot) {
-        const int ks = min(kt, p.nk - 1);
+        const int ks = min(kt, kt1 - 1);
         const unsigned base = sm0 + (unsigned)(slot * STAGE);
 #pragma unroll
         for (int j = 0; j < L; j++) {
@@ -793,10 +815,10 @@ __global__ __launch_bounds__(ring::T, 1) void k_gemm_ring(GemmP p) {
         for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     ring_wait<0>();
 #pragma unroll
-    for (int s = 0; s < S - 1; s++) issue(s, s);
+    for (int s = 0; s < S - 1; s++) issue(kt0 + s, s);
     const int fr = lane & 15, g = lane >> 4;
     int cur = 0;  // ring slot of step kt
-    for (int kt = 0; kt < p.nk; kt++) {
+    for (int kt = kt0; kt < kt1; kt++) {
         ring_wait<L * (S - 2)>();  // this wave's loads of step kt have landed
         ring_barrier();            // every wave's have; slot kt - 1 is free
         issue(kt + S - 1, cur == 0 ? S - 1 : cur - 1);
@@ -841,12 +863,43 @@ __global__ __launch_bounds__(ring::T, 1) void k_gemm_ring(GemmP p) {
         }
     }
     ring_wait<0>();  // the re-read tail steps land before the workgroup's LDS is reused or released
+    if (!C::BIG && p.splits > 1) {
+        float *part = p.partf + (size_t)sp * p.M * p.N;
+#pragma unroll
+        for (int tn = 0; tn < TN; tn++) {
+            const int n = n0 + wn * TN * 16 + tn * 16 + fr;
+#pragma unroll
+            for (int tm = 0; tm < TM; tm++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int m = m0 + wm * TM * 16 + tm * 16 + (g << 2) + r;
+                    if (m < p.M && n < p.N) part[(size_t)m * p.N + n] = acc[tm][tn][r];
+                }
+        }
+        return;
+    }
     if (EPI == GE_SWIGLU) {
         __syncthreads();  // every wave's tail loads have landed
-        swiglu_store<TM, TN, T, WBF>(p, acc, reinterpret_cast<u16 *>(sm), wm * TM * 16, wn * TN * 16, m0, n0, lane);
-        if (wave == 0 && nbk == p.n_nb - 1) swiglu_pad(p, m0, lane);
+        swiglu_store<TM, TN, T, WBF, C::BM, C::BN>(p, acc, reinterpret_cast<u16 *>(sm), wm * TM * 16, wn * TN * 16, m0,
+                                                   n0, lane);
+        if (wave == 0 && nbk == p.n_nb - 1) swiglu_pad<C::BM>(p, m0, lane);
     } else {
         gemm_store<EPI, TM, TN>(p, acc, m0 + wm * TM * 16, n0 + wn * TN * 16, lane, p.scale, p.scale2);
+    }
+}
+
+// The k splits' f32 sums of k_gemm_ring, added in split order, then
+// gemm_store's epilogue.
+template <int EPI>
+__global__ __launch_bounds__(256) void k_ring_finish(GemmP p) {
+    const size_t mn = (size_t)p.M * p.N;
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < mn; t += (size_t)gridDim.x * 256) {
+        const int m = (int)(t / p.N), n = (int)(t % p.N);
+        float v = p.partf[t];
+        for (int sp = 1; sp < p.splits; sp++) v += p.partf[(size_t)sp * mn + t];
+        v *= p.scale;
+        float *c = p.c + (size_t)m * p.ldc + n;
+        *c = EPI == GE_RESID ? *c + v : p.bias ? v + p.bias[n] : v;
     }
 }
 
@@ -888,19 +941,6 @@ struct DTile {
 using DBig = DTile<BM, BN, 2, 4, 3>;
 static_assert(DBig::LDS >= 2 * BM * (BN / 2 + 8) * sizeof(u16), "SwiGLU plane staging tile");
 
-// Workgroup -> (tile, k split) of the smaller tiles: XCD b % 8 walks a
-// contiguous run, row tiles fastest, so the row tiles of one weight panel
-// share an L2 (the super-tile map would leave XCDs without work here).
-__device__ __forceinline__ bool digit_tile(const GemmP &p, int &mb, int &nb, int &sp) {
-    const unsigned total = (unsigned)p.n_mb * p.n_nb * p.splits, per = (total + 7) / 8;
-    const unsigned w = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((blockIdx.x >> 3) >= per || w >= total) return false;
-    mb = (int)(w % p.n_mb);
-    nb = (int)(w / p.n_mb % p.n_nb);
-    sp = (int)(w / ((unsigned)p.n_mb * p.n_nb));
-    return true;
-}
-
 // S 2^-E scale in f64, one rounding to f32
 __device__ __forceinline__ float digit_value(double S, int E, double sc) {
     return E == DG_NONFINITE ? __builtin_nanf("") : (float)(S * ldexp(1.0, -E) * sc);
@@ -914,7 +954,7 @@ __global__ __launch_bounds__(TL::T, TL::BIG ? 1 : 2) void k_gemm_digits(GemmP p)
     extern __shared__ float4 dsm[];
     unsigned char *sm = reinterpret_cast<unsigned char *>(dsm);
     int mb, nbk, sp = 0;
-    if (TL::BIG ? !gemm_tile(p, mb, nbk) : !digit_tile(p, mb, nbk, sp)) return;
+    if (TL::BIG ? !gemm_tile(p, mb, nbk) : !small_tile(p, mb, nbk, sp)) return;
     const int m0 = mb * TL::BM, n0 = nbk * TL::BN;
     // this split's k steps
     const int kt0 = TL::BIG ? 0 : sp * p.kchunk, kt1 = TL::BIG ? p.nk : min(p.nk, kt0 + p.kchunk);
@@ -1032,7 +1072,7 @@ __global__ __launch_bounds__(TL::T, TL::BIG ? 1 : 2) void k_gemm_digits(GemmP p)
         __syncthreads();  // every wave's tail loads have landed
         swiglu_store<TM, TN, T, false, TL::BM, TL::BN>(q, v, reinterpret_cast<u16 *>(sm), wm * TM * 16, wn * TN * 16, m0,
                                                        n0, lane);
-        if (TL::BIG && !p.of && wave == 0 && nbk == p.n_nb - 1) swiglu_pad(p, m0, lane);
+        if (TL::BIG && !p.of && wave == 0 && nbk == p.n_nb - 1) swiglu_pad<BM>(p, m0, lane);
     } else {
         gemm_store<EPI, TM, TN>(q, v, m0 + wm * TM * 16, n0 + wn * TN * 16, lane, 1.f, 1.f);
     }
@@ -1678,29 +1718,35 @@ int digits_small(GemmP p, int splits, hipStream_t s) {
 // Tile and k splits for M rows.  The time of a choice: k steps of a split times
 // the workgroups each CU runs one after another or together (workgroups / 256)
 // times the measured time of one workgroup's step (us, from 17-1024 rows at
-// k 768-11008, n 768-22016: alone on a CU / sharing it), plus the f64 partial
-// sums' round trip.  Measured, old tile -> this choice: 512 x 11008 x 4096
-// (rows, k, n) 193 -> 91 us, 512 x 4096 x 4096 81 -> 43, 130 x 4096 x 14336
-// 80 -> 57, 64 x 11008 x 4096 180 -> 29, 200 x 768 x 2304 26 -> 11; from about
-// 224 tiles of 128 x 256 on the large tile stays the fastest (512 x 4096 x
-// 14336: 89 us against 113, 1024 x 4096 x 22016: 245 against 324).
-struct DigitPick {
+// k 768-11008, n 768-28672: alone on a CU / sharing it), plus the partial
+// sums' round trip.  From about 224 tiles of 128 x 256 on the large tile stays
+// the fastest.  Measured, that tile -> this choice (rows x k x n):
+//   digits  512 x 11008 x 4096 193 -> 91 us, 512 x 4096 x 4096 81 -> 43, 130 x
+//           4096 x 14336 80 -> 57, 64 x 11008 x 4096 180 -> 29, 200 x 768 x
+//           2304 26 -> 11; kept: 512 x 4096 x 14336 89 (next best 113)
+//   bf16    512 x 11008 x 4096 180 -> 65, 37 x 4096 x 12288 63 -> 22, 37 x
+//           11008 x 4096 152 -> 22, 130 x 4096 x 28672 134 -> 81, 256 x 768 x
+//           2304 22 -> 8; kept: 512 x 4096 x 28672 157 (next best 188)
+struct TileCost {
+    int bm, bn;
+    double alone, shared;
+};
+constexpr TileCost kDigitTiles[5] = {{128, 256, 1.25, 1.25}, {128, 128, 0.80, 0.80}, {64, 128, 0.52, 0.50}, {64, 64, 0.38, 0.345}, {32, 128, 0.376, 0.34}};
+constexpr TileCost kRingTiles[5] = {{128, 256, 1.15, 1.20}, {128, 128, 0.65, 0.70}, {64, 128, 0.42, 0.36}, {64, 64, 0.33, 0.23}, {32, 128, 0.34, 0.26}};
+struct TilePick {
     int tile, splits;
 };
-DigitPick pick_digits(int M, int N, int nk, bool small_ok) {
-    struct {
-        int bm, bn;
-        double alone, shared;
-    } const tl[] = {{128, 256, 1.25, 1.25}, {128, 128, 0.80, 0.80}, {64, 128, 0.52, 0.50}, {64, 64, 0.38, 0.345}, {32, 128, 0.376, 0.34}};
-    DigitPick best{0, 1};
+TilePick pick_tile(const TileCost (&tl)[5], int M, int N, int nk, int part_bytes, int n_tiles, int max_splits) {
+    TilePick best{0, 1};
     double bt = 1e30;
-    for (int i = 0; i < (small_ok ? 5 : 1); i++) {
+    for (int i = 0; i < n_tiles; i++) {
         const double tiles = (double)((M + tl[i].bm - 1) / tl[i].bm) * ((N + tl[i].bn - 1) / tl[i].bn);
-        for (int sp = 1; sp <= (i ? 16 : 1); sp *= 2) {
-            if (sp > 1 && (nk < 4 * sp || (double)sp * M * N > 33554432.0)) break;  // at most 256 MB of partials
+        for (int sp = 1; sp <= (i ? max_splits : 1); sp *= 2) {
+            const double bytes = (double)sp * M * N * part_bytes;
+            if (sp > 1 && (nk < 4 * sp || bytes > 268435456.0)) break;  // at most 256 MB of partial sums
             const double n = std::ceil(tiles * sp / 256.0);
             double t = (nk + sp - 1) / sp * n * (n > 1 ? tl[i].shared : tl[i].alone);
-            if (sp > 1) t += 4.0 + (double)sp * M * N * 16.0 / 5.0e6;
+            if (sp > 1) t += 4.0 + 2.0 * bytes / 5.0e6;
             if (t < bt) bt = t, best = {i, sp};
         }
     }
@@ -1710,7 +1756,7 @@ DigitPick pick_digits(int M, int N, int nk, bool small_ok) {
 template <int EPI>
 int gemm_digits_t(const GemmP &p, hipStream_t s) {
     // the smaller tiles write SwiGLU as f32 rows only
-    const DigitPick d = pick_digits(p.M, p.N, p.nk, EPI != GE_SWIGLU || p.of);
+    const TilePick d = pick_tile(kDigitTiles, p.M, p.N, p.nk, sizeof(double), EPI != GE_SWIGLU || p.of ? 5 : 1, 16);
     switch (d.tile) {
         case 1: return digits_small<EPI, DTile<128, 128, 2, 4, 3>>(p, d.splits, s);
         case 2: return digits_small<EPI, DTile<64, 128, 2, 2, 3>>(p, d.splits, s);
@@ -1720,18 +1766,51 @@ int gemm_digits_t(const GemmP &p, hipStream_t s) {
     return digits_launch<EPI, DBig>(p, (p.n_super + 7) / 8 * 8 * 32, s);
 }
 
-template <int EPI, bool WBF>
-int gemm_ring_t(const GemmP &p, hipStream_t s) {
-    constexpr size_t lds = ring::Lay<WBF>::LDS;
+template <int EPI, bool WBF, class C>
+int ring_launch(const GemmP &p, int grid, hipStream_t s) {
     static bool attr = false;
     if (!attr) {
-        SCRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gemm_ring<EPI, WBF>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        SCRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gemm_ring<EPI, WBF, C>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS));
         attr = true;
     }
-    const int grid = (p.n_super + 7) / 8 * 8 * 32;
-    hipLaunchKernelGGL((k_gemm_ring<EPI, WBF>), dim3(grid), dim3(ring::T), lds, s, p);
+    hipLaunchKernelGGL((k_gemm_ring<EPI, WBF, C>), dim3(grid), dim3(C::T), C::LDS, s, p);
     PF_LAUNCH_CHECK();
+}
+
+template <int EPI, class C>
+int ring_small(GemmP p, int splits, hipStream_t s) {
+    p.n_mb = (p.M + C::BM - 1) / C::BM;
+    p.n_nb = (p.N + C::BN - 1) / C::BN;
+    p.kchunk = (p.nk + splits - 1) / splits;
+    p.splits = (p.nk + p.kchunk - 1) / p.kchunk;
+    if (p.splits > 1) {
+        void *ws = nullptr;
+        SCRY_TRY(ctx_workspace(sizeof(float) * (size_t)p.splits * p.M * p.N, &ws));
+        p.partf = (float *)ws;
+    }
+    SCRY_TRY((ring_launch<EPI, true, C>(p, (p.n_mb * p.n_nb * p.splits + 7) / 8 * 8, s)));
+    if (p.splits > 1) {
+        const size_t g = ((size_t)p.M * p.N + 255) / 256;
+        hipLaunchKernelGGL(k_ring_finish<EPI>, dim3((unsigned)std::min<size_t>(g, 65536)), dim3(256), 0, s, p);
+        PF_LAUNCH_CHECK();
+    }
+    return SCRY_OK;
+}
+
+template <int EPI, bool WBF>
+int gemm_ring_t(const GemmP &p, hipStream_t s) {
+    if constexpr (WBF) {
+        // SwiGLU planes come from the whole sums: no k splits
+        const TilePick d = pick_tile(kRingTiles, p.M, p.N, p.nk, sizeof(float), 5, EPI == GE_SWIGLU ? 1 : 8);
+        switch (d.tile) {
+            case 1: return ring_small<EPI, RTile<true, 128, 128, 2, 4, 3>>(p, d.splits, s);
+            case 2: return ring_small<EPI, RTile<true, 64, 128, 2, 2, 3>>(p, d.splits, s);
+            case 3: return ring_small<EPI, RTile<true, 64, 64, 2, 2, 4>>(p, d.splits, s);
+            case 4: return ring_small<EPI, RTile<true, 32, 128, 1, 4, 4>>(p, d.splits, s);
+        }
+    }
+    return ring_launch<EPI, WBF, RBig<WBF>>(p, (p.n_super + 7) / 8 * 8 * 32, s);
 }
 
 }  // namespace

@@ -55,3 +55,41 @@ def test_prefill_with_split_k_matches_decode(hip, seq):
         ref, _ = m.forward_with_llama_cache(int(t), p, cd)
     assert np.abs(last - ref).max() <= 1e-3 * np.abs(ref).max()
     m.free()
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (17, 64, 5), (37, 100, 131), (32, 4096, 260), (64, 768, 768), (130, 4096, 1030), (200, 3072, 770),
+    (129, 1280, 5120), (300, 1024, 4097), (512, 8192, 1024)])
+def test_bf16_exact_sums(hip, m, k, n):
+    """The bf16 GEMM's tiles and splits: integers exact in bf16, sums exact in f32."""
+    print(f"[case] bf16 {m} x {k} x {n}", flush=True)
+    B = hip.HipBackend
+    rng = np.random.default_rng(m + k + n)
+    a = rng.integers(-8, 9, (m, k)).astype(F)
+    w = rng.integers(-64, 65, (k, n)).astype(F)
+    ref = a.astype(np.float64) @ w.astype(np.float64)
+    B.set_bf16_mode(True)
+    try:
+        c = B.matmul(B.from_vec(a), B.from_vec(w), m, k, n).to_vec().reshape(m, n)
+    finally:
+        B.set_bf16_mode(False)
+    assert np.array_equal(c, ref)
+
+
+@pytest.mark.parametrize("seq", [18, 70, 130])
+def test_bf16_prefill_small_tiles_match_decode(hip, seq):
+    """The residual splits and the SwiGLU planes of the smaller bf16 tiles, against
+    the decode path (both round activations to bf16; one rounding apart at most
+    per value: 1e-2 as the bf16 model's other prefill tests)."""
+    print(f"[case] bf16 seq={seq}", flush=True)
+    import esolearn_amd.llama as EL
+    cfg = hip.LlamaConfig(vocab_size=96, hidden_size=2048, intermediate_size=4104, n_layers=1, n_heads=16,
+                          n_kv_heads=4, max_seq_len=256, rope_theta=10000.0, tie_word_embeddings=False)
+    m = hip.LlamaModel.new_random(cfg, 3, quant_mode=EL.QUANT_BF16, init_on_device=True)
+    toks = np.random.default_rng(seq).integers(0, 96, seq)
+    cp, cd = m.new_llama_kv_cache(seq), m.new_llama_kv_cache(seq)
+    last = m.prefill([cp], toks[None, :])[0]
+    for p, t in enumerate(toks):
+        ref, _ = m.forward_with_llama_cache(int(t), p, cd)
+    assert np.abs(last - ref).max() <= 1e-2 * np.abs(ref).max()
+    m.free()

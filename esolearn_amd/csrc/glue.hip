@@ -59,6 +59,17 @@ __global__ void k_rope(const float *__restrict__ x, int seq, int n_heads, int hd
     }
 }
 
+// A cache's RoPE table (cpu.rs:648-652).  Bound by the f64 cos / sin; on the
+// host this table was 1 ms per 1000 positions and cache (4 caches of 1031
+// positions: 4.1 of a 14 ms batch), here a few us.
+__global__ void k_rope_table(const float *__restrict__ freqs, int n_pos, int half, float2 *__restrict__ cs) {
+    const size_t total = (size_t)n_pos * half;
+    GRID_STRIDE(t, total) {
+        const double ang = (double)(t / half) * (double)freqs[t % half];
+        cs[t] = make_float2((float)cos(ang), (float)sin(ang));
+    }
+}
+
 __global__ void k_scale(const float *__restrict__ x, size_t n, float s, float *__restrict__ out) {
     GRID_STRIDE(i, n) out[i] = __fmul_rn(x[i], s);
 }
@@ -220,6 +231,13 @@ int launch_rope(const float *x, int seq, int n_heads, int hd, int start_pos, con
     if (total == 0) return SCRY_OK;
     hipLaunchKernelGGL(k_rope, dim3(grid1(total)), dim3(256), 0, s, x, seq, n_heads, hd, start_pos,
                        freqs, scaled, scale, out);
+    LAUNCH_CHECK();
+}
+
+int launch_rope_table(const float *freqs, int n_pos, int half, float2 *cs, hipStream_t s) {
+    const size_t total = (size_t)n_pos * half;
+    if (total == 0) return SCRY_OK;
+    hipLaunchKernelGGL(k_rope_table, dim3(grid1(total)), dim3(256), 0, s, freqs, n_pos, half, cs);
     LAUNCH_CHECK();
 }
 

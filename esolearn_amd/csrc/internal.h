@@ -274,6 +274,8 @@ int launch_rmsnorm(const float *x, const float *w, int rows, int d, float eps, f
                    hipStream_t s);
 int launch_rope(const float *x, int seq, int n_heads, int hd, int start_pos, const float *freqs,
                 int scaled, float scale, float *out, hipStream_t s);
+// cs[p][i] = (cos, sin) of f64(p) * f64(freqs[i]), rounded to f32
+int launch_rope_table(const float *freqs, int n_pos, int half, float2 *cs, hipStream_t s);
 int launch_scale(const float *x, size_t n, float s_, float *out, hipStream_t s);
 int launch_softmax(const float *x, int rows, int cols, float *out, hipStream_t s);
 int launch_swiglu(const float *g, const float *u, size_t n, float *out, hipStream_t s);

@@ -42,6 +42,7 @@ struct scry_llama_s {
     // config.rms_norm_eps; a loaded checkpoint uses the config's (llama.rs:880-914)
     float eps = 1e-5f;
     std::vector<float> freqs;  // [hd/2] f32 (llama.rs:618-622)
+    float *freqs_d = nullptr;  // the same on the device (cache_new's table kernel)
     struct Layer {
         Packed qkv, o, gu, down;
     };
@@ -97,7 +98,7 @@ struct scry_kv_cache_s {
     int max_seq = 0;
     int seq_len = 0;  // host mirror of LlamaLayerKvCache::seq_len
     float *kv = nullptr;  // [L][2][max_seq][kv_dim]
-    float2 *rope_cs = nullptr;  // [max_seq][hd/2] (cos, sin), glibc values as cpu.rs:650-652
+    float2 *rope_cs = nullptr;  // [max_seq][hd/2] (cos, sin) as cpu.rs:650-652
     DevState *state = nullptr;
     int64_t *tokens = nullptr;
     int tokens_len = 0;
@@ -250,6 +251,7 @@ void model_free(scry_llama m) {
     packed_free(m->lm);
     dev_free(m->embed);
     dev_free(m->norms);
+    dev_free(m->freqs_d);
     dev_free(m->bits);
     dev_free(m->stage);
     dev_free(m->pf.p0);
@@ -323,6 +325,13 @@ int model_alloc(const scry_llama_config *cfg, int quant_mode, scry_llama *out) {
     int rc = dev_alloc((void **)&m->embed, sizeof(float) * (size_t)m->V * h);
     if (!rc) rc = dev_alloc((void **)&m->norms, sizeof(float) * (size_t)(2 * m->L + 1) * h);
     if (!rc) rc = launch_fill_f32(m->norms, (size_t)(2 * m->L + 1) * h, 1.0f, ctx().stream);
+    if (!rc) rc = dev_alloc((void **)&m->freqs_d, sizeof(float) * m->freqs.size());
+    if (!rc && !m->freqs.empty()) {
+        hipError_t e = hipMemcpyAsync(m->freqs_d, m->freqs.data(), sizeof(float) * m->freqs.size(),
+                                      hipMemcpyHostToDevice, ctx().stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(ctx().stream);
+        if (e != hipSuccess) rc = hip_fail(e, "rope frequencies upload", __FILE__, __LINE__);
+    }
     if (!rc) rc = dev_alloc((void **)&m->bits, 16);
     const size_t sizes[] = {(size_t)m->V * h, (size_t)h * m->qkv_dim, (size_t)h * m->ffn,
                             (size_t)m->q_dim * h};
@@ -421,21 +430,7 @@ int cache_new(scry_llama m, int max_seq, scry_kv_cache *out) {
         hipError_t e = hipHostMalloc((void **)&c->hs, sizeof(HostStage), hipHostMallocDefault);
         if (e != hipSuccess) rc = hip_fail(e, "hipHostMalloc", __FILE__, __LINE__);
     }
-    if (!rc) {
-        // RoPE table: cos/sin of f64(pos) * f64(freq_f32) rounded to f32, with
-        // the host libm the reference uses (cpu.rs:648-652)
-        const int hh = m->hd / 2;
-        std::vector<float2> cs((size_t)max_seq * hh);
-        for (int p = 0; p < max_seq; p++)
-            for (int i = 0; i < hh; i++) {
-                const double ang = (double)p * (double)m->freqs[i];
-                cs[(size_t)p * hh + i] = make_float2((float)std::cos(ang), (float)std::sin(ang));
-            }
-        hipError_t e = hipMemcpyAsync(c->rope_cs, cs.data(), sizeof(float2) * cs.size(),
-                                      hipMemcpyHostToDevice, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) rc = hip_fail(e, "rope table upload", __FILE__, __LINE__);
-    }
+    if (!rc) rc = launch_rope_table(m->freqs_d, max_seq, m->hd / 2, c->rope_cs, s);
     if (rc) {
         cache_free(c);
         return rc;

@@ -880,6 +880,19 @@ int prefill_core(scry_llama m, scry_kv_cache *cs, int n_seq, const int64_t *toke
                 g.y = last_logits + (size_t)i * m->V;
                 SCRY_TRY(launch_qgemv(EPI_STORE, g, s));
             }
+        } else if (skinny_route(n_seq, m->h, m->lm.rows)) {
+            // the op-level matmul's route: several rows on the matrix cores (4
+            // rows x 128256 columns: 229 us as a GEMV over 4 rows)
+            void *ws = nullptr;
+            SCRY_TRY(ctx_workspace(skinny_ws_bytes(n_seq, m->h, m->lm.rows), &ws));
+            SkinnyMM sm;
+            sm.w = &m->lm;
+            sm.x = P.xl;
+            sm.ldx = m->h;
+            sm.m = n_seq;
+            sm.y = last_logits;
+            sm.ldy = m->V;
+            SCRY_TRY(launch_skinny(sm, (float *)ws, ctx().ws_bytes, s));
         } else {
             SCRY_TRY(launch_qgemv(EPI_STORE, g, s));
         }

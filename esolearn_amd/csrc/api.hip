@@ -898,8 +898,8 @@ int scry_hip_argmax(scry_buf logits, int64_t *out) {
     CHECK_BUF(logits, "argmax");
     if (!out) return set_error(SCRY_ERR_INVALID, "argmax: null output");
     int64_t *d = nullptr;
-    SCRY_TRY(pool_alloc((void **)&d, sizeof(int64_t)));
-    int rc = launch_argmax(logits->d, (int64_t)logits->n, d, ctx().stream);
+    SCRY_TRY(pool_alloc((void **)&d, sizeof(int64_t) * 2 + kArgmaxScratch));
+    int rc = launch_argmax(logits->d, (int64_t)logits->n, d, d + 2, ctx().stream);
     if (!rc) {
         hipError_t e = hipMemcpyAsync(out, d, sizeof(int64_t), hipMemcpyDeviceToHost, ctx().stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx().stream);

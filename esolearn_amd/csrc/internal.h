@@ -291,7 +291,8 @@ int launch_repeat_kv(const float *x, int n_kv, int n_q, int seq, int d_head, flo
 // added in f32
 int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, int n, int ta, int tb,
                       const float *bias, float *c, hipStream_t s);
-int launch_argmax(const float *x, int64_t n, int64_t *out, hipStream_t s);
+constexpr size_t kArgmaxScratch = 4096;  // bytes of device scratch launch_argmax needs (`part`)
+int launch_argmax(const float *x, int64_t n, int64_t *out, void *part, hipStream_t s);
 int launch_fill_f32(float *p, size_t n, float v, hipStream_t s);
 int launch_fill_u32(unsigned int *p, size_t n, unsigned int v, hipStream_t s);
 // Rows of int8 LM-head logits whose RMSNorm'd input holds a non-finite value:

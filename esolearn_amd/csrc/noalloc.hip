@@ -78,7 +78,8 @@ extern "C" int scry_hip_sample_token_noalloc(scry_buf logits, const scry_samplin
     static_assert(sizeof(DevState) == 16, "DevState layout");
     static_assert(sizeof(h) <= NA_HDR, "scratch header");
     if (cfg->temperature < 1e-8f) {  // generate.rs:96-98: argmax, no draw
-        SCRY_TRY(launch_argmax(logits->d, (int64_t)V, toks + 1, s));
+        static_assert(sizeof(double) * NA_MAX_V >= kArgmaxScratch, "argmax scratch");
+        SCRY_TRY(launch_argmax(logits->d, (int64_t)V, toks + 1, ws, s));
         SCRY_HIP(hipMemcpyAsync(&h.toks[1], toks + 1, sizeof(int64_t), hipMemcpyDeviceToHost, s));
         SCRY_HIP(hipStreamSynchronize(s));
         *out = h.toks[1];

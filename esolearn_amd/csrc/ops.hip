@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "kdev.h"
 
 #pragma clang fp contract(off)
 
@@ -57,6 +58,67 @@ __global__ __launch_bounds__(256) void k_layernorm(const float *__restrict__ x, 
         out[(size_t)blockIdx.x * d + j] = (float)(nrm * (double)g[j] + (double)b[j]);
     }
     if (threadIdx.x == 0 && mean_out) {
+        mean_out[blockIdx.x] = (float)mean;
+        rstd_out[blockIdx.x] = (float)rstd;
+    }
+}
+
+// The same with the row read once, 16 bytes per load, and kept in registers
+// (d % 4 == 0, d <= 4 NT NV).  A wave per row from 256 rows on (no barriers:
+// 1500 x 1280 11.5 us as a workgroup of 256 with either kernel, 8.6 so), else
+// enough threads for one value quad each (a row's latency is the kernel).
+template <int NT, int NV>
+__global__ __launch_bounds__(NT) void k_layernorm4(const float4 *__restrict__ x, const float4 *__restrict__ g,
+                                                   const float4 *__restrict__ b, int d4, float eps,
+                                                   float4 *__restrict__ out, float *__restrict__ mean_out,
+                                                   float *__restrict__ rstd_out) {
+    __shared__ double red[2][NT / 64];
+    const float4 *r = x + (size_t)blockIdx.x * d4;
+    const int tid = threadIdx.x;
+    float4 v[NV], gv[NV], bv[NV];
+#pragma unroll
+    for (int c = 0; c < NV; c++) {
+        const int j = c * NT + tid;
+        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+        v[c] = j < d4 ? r[j] : z;
+        gv[c] = j < d4 ? g[j] : z;
+        bv[c] = j < d4 ? b[j] : z;
+    }
+    auto total = [&](double s, double *sh) {
+        s = dev::wave_sum_d_dpp(s);
+        if (NT == 64) return s;
+        if ((tid & 63) == 0) sh[tid >> 6] = s;
+        __syncthreads();
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < NT / 64; i++) t += sh[i];
+        return t;
+    };
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < NV; c++) s += ((double)v[c].x + (double)v[c].y) + ((double)v[c].z + (double)v[c].w);
+    const double mean = total(s, red[0]) / (double)(4 * d4);
+    double q = 0.0;
+#pragma unroll
+    for (int c = 0; c < NV; c++) {
+        if (c * NT + tid < d4) {
+            const double a = v[c].x - mean, e = v[c].y - mean, f = v[c].z - mean, h = v[c].w - mean;
+            q += (a * a + e * e) + (f * f + h * h);
+        }
+    }
+    const double rstd = 1.0 / sqrt(total(q, red[1]) / (double)(4 * d4) + (double)eps);
+    auto one = [&](float xv, float ga, float be) {
+        return (float)(((double)xv - mean) * rstd * (double)ga + (double)be);
+    };
+#pragma unroll
+    for (int c = 0; c < NV; c++) {
+        const int j = c * NT + tid;
+        if (j < d4)
+            out[(size_t)blockIdx.x * d4 + j] =
+                make_float4(one(v[c].x, gv[c].x, bv[c].x), one(v[c].y, gv[c].y, bv[c].y),
+                            one(v[c].z, gv[c].z, bv[c].z), one(v[c].w, gv[c].w, bv[c].w));
+    }
+    if (tid == 0 && mean_out) {
         mean_out[blockIdx.x] = (float)mean;
         rstd_out[blockIdx.x] = (float)rstd;
     }
@@ -116,13 +178,27 @@ __global__ void k_rope_row(const float *__restrict__ x, size_t rows, int last_di
     }
 }
 
-// mod.rs:316-331 gather_columns: out[r][c] = x[r][start + c]
+// W values (16 bytes for 4) moved as one access
+template <int W>
+struct Vals {
+    float v[W];
+};
+template <>
+struct __align__(16) Vals<4> {
+    float v[4];
+};
+
+// mod.rs:316-331 gather_columns: out[r][c] = x[r][start + c] (W = 4: all of
+// them multiples of 4)
+template <int W>
 __global__ void k_gather_cols(const float *__restrict__ x, size_t rows, int total, int start, int count,
                               float *__restrict__ out) {
-    const size_t n = rows * (size_t)count;
+    const unsigned cw = (unsigned)count / W;
+    const size_t n = rows * cw;
     GRID_STRIDE(t, n) {
-        const size_t r = t / count;
-        out[t] = x[r * total + start + (t % count)];
+        const size_t r = t / cw;
+        reinterpret_cast<Vals<W> *>(out)[t] =
+            *reinterpret_cast<const Vals<W> *>(x + r * total + start + (t % cw) * W);
     }
 }
 
@@ -164,78 +240,68 @@ __global__ void k_add_inplace(float *__restrict__ d, const float *__restrict__ s
     GRID_STRIDE(i, n) d[i] = d[i] + s[i];
 }
 
-// cpu.rs:300-334 scaled_softmax: v = x * scale (f32), max of v, e = expf(v - max)
-// kept as f32, f64 sum, out = f32(f64(e) / sum).  One workgroup per row.
-__global__ __launch_bounds__(256) void k_scaled_softmax(const float *__restrict__ x, int cols, float scale,
-                                                        float *__restrict__ out) {
-    const float *r = x + (size_t)blockIdx.x * cols;
-    float *o = out + (size_t)blockIdx.x * cols;
-    __shared__ float redf[4];
-    __shared__ double redd[4];
-    float mx = -INFINITY;
-    for (int j = threadIdx.x; j < cols; j += 256) mx = fmaxf(mx, r[j] * scale);
-    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-    if ((threadIdx.x & 63) == 0) redf[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
-    double sum = 0.0;
-    for (int j = threadIdx.x; j < cols; j += 256) {
-        const float e = expf(r[j] * scale - mx);
-        o[j] = e;
-        sum += (double)e;
-    }
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-    if ((threadIdx.x & 63) == 0) redd[threadIdx.x >> 6] = sum;
-    __syncthreads();
-    sum = (redd[0] + redd[1]) + (redd[2] + redd[3]);
-    for (int j = threadIdx.x; j < cols; j += 256) o[j] = (float)((double)o[j] / sum);
-}
-
 // mod.rs:384-401 / 595-621: t > s -> mask_value, else *= scale, on n_mat
-// [seq, seq] matrices in place
-__global__ void k_causal_mask(float *__restrict__ sc, size_t n_mat, int seq, float scale, float mask_value) {
-    const size_t mat = (size_t)seq * seq, n = n_mat * mat;
-    GRID_STRIDE(t, n) {
-        const size_t w = t % mat;
-        const int s = (int)(w / seq), c = (int)(w % seq);
-        sc[t] = c > s ? mask_value : sc[t] * scale;
+// [seq, seq] matrices in place.  A workgroup takes rows blockIdx.x, + gridDim.x
+// ...; values above the diagonal are not read (32 x 512 x 512: 20 -> 17 us).
+// W = 4 (seq % 4 == 0): 16-byte accesses.
+template <int W>
+__global__ __launch_bounds__(256) void k_causal_mask(float *__restrict__ sc, size_t n_rows, int seq, float scale,
+                                                     float mask_value) {
+    for (size_t row = blockIdx.x; row < n_rows; row += gridDim.x) {
+        const int s = (int)(row % seq);
+        float *p = sc + row * seq;
+        for (int c = (int)threadIdx.x * W; c < seq; c += 256 * W) {
+            Vals<W> v;
+            if (c <= s) v = *reinterpret_cast<const Vals<W> *>(p + c);
+#pragma unroll
+            for (int e = 0; e < W; e++) v.v[e] = c + e > s ? mask_value : v.v[e] * scale;
+            *reinterpret_cast<Vals<W> *>(p + c) = v;
+        }
     }
 }
 
-// mod.rs:408-438 split_qkv_reshape_heads: [seq, 3 d_model] -> three
-// [n_heads, seq, d_head]
+// mod.rs:408-438 split_qkv_reshape_heads: [seq, 3*d_model] -> three
+// [n_heads, seq, d_head]; W values per access (4 where d_head % 4 == 0)
+template <int W>
 __global__ void k_split_qkv(const float *__restrict__ qkv, int seq, int n_heads, int d_head,
                             float *__restrict__ q, float *__restrict__ k, float *__restrict__ v) {
-    const int dm = n_heads * d_head;
-    const size_t n = (size_t)seq * dm;
-    GRID_STRIDE(t, n) {  // t = (h * seq + s) * d_head + d
-        const int d = (int)(t % d_head);
-        const size_t hs = t / d_head;
+    typedef Vals<W> T;
+    const int dw = d_head / W;
+    const size_t dm = (size_t)n_heads * dw, n = (size_t)seq * dm;  // in accesses
+    const T *src = reinterpret_cast<const T *>(qkv);
+    GRID_STRIDE(t, n) {  // t = (h * seq + s) * dw + d
+        const int d = (int)(t % dw);
+        const size_t hs = t / dw;
         const int s = (int)(hs % seq), h = (int)(hs / seq);
-        const size_t row = (size_t)s * 3 * dm + (size_t)h * d_head + d;
-        q[t] = qkv[row];
-        k[t] = qkv[row + dm];
-        v[t] = qkv[row + 2 * dm];
+        const size_t row = (size_t)s * 3 * dm + (size_t)h * dw + d;
+        reinterpret_cast<T *>(q)[t] = src[row];
+        reinterpret_cast<T *>(k)[t] = src[row + dm];
+        reinterpret_cast<T *>(v)[t] = src[row + 2 * dm];
     }
 }
 
 // mod.rs:441-467 reshape_for_heads: [B*S, H*d] -> [B*H, S, d] (dir 0) and
 // mod.rs:484-510 reshape_from_heads, its inverse (dir 1)
+template <int W>
 __global__ void k_reshape_heads(const float *__restrict__ x, int batch, int seq, int n_heads, int d_head, int dir,
                                 float *__restrict__ out) {
-    const size_t n = (size_t)batch * seq * n_heads * d_head;
+    typedef Vals<W> T;
+    const int dw = d_head / W;
+    const size_t n = (size_t)batch * seq * n_heads * dw;
+    const T *src = reinterpret_cast<const T *>(x);
+    T *dst = reinterpret_cast<T *>(out);
     GRID_STRIDE(t, n) {  // t indexes the [B*H, S, d] layout
-        const int d = (int)(t % d_head);
-        const size_t r = t / d_head;
+        const int d = (int)(t % dw);
+        const size_t r = t / dw;
         const int s = (int)(r % seq);
         const size_t bh = r / seq;
         const int h = (int)(bh % n_heads);
         const size_t b = bh / n_heads;
-        const size_t flat = ((b * seq + s) * n_heads + h) * d_head + d;  // [B*S, H*d] index
+        const size_t flat = ((b * seq + s) * n_heads + h) * dw + d;  // [B*S, H*d] index
         if (dir == 0)
-            out[t] = x[flat];
+            dst[t] = src[flat];
         else
-            out[flat] = x[t];
+            dst[flat] = src[t];
     }
 }
 
@@ -246,7 +312,18 @@ __global__ void k_reshape_heads(const float *__restrict__ x, int batch, int seq,
 int launch_layernorm(const float *x, const float *g, const float *b, int rows, int d, float eps, float *out,
                      float *mean, float *rstd, hipStream_t s) {
     if (rows <= 0 || d <= 0) return SCRY_OK;
-    hipLaunchKernelGGL(k_layernorm, dim3(rows), dim3(256), 0, s, x, g, b, d, eps, out, mean, rstd);
+    const bool v4 = d % 4 == 0 && ((uintptr_t)x | (uintptr_t)g | (uintptr_t)b | (uintptr_t)out) % 16 == 0;
+    const int d4 = d / 4;
+#define LN4(NT, NV)                                                                                             \
+    hipLaunchKernelGGL((k_layernorm4<NT, NV>), dim3(rows), dim3(NT), 0, s, (const float4 *)x, (const float4 *)g, \
+                       (const float4 *)b, d4, eps, (float4 *)out, mean, rstd)
+    if (v4 && rows >= 256 && d4 <= 256) LN4(64, 4);
+    else if (v4 && rows >= 256 && d4 <= 512) LN4(64, 8);
+    else if (v4 && d4 <= 256) LN4(256, 1);
+    else if (v4 && d4 <= 1024) LN4(1024, 1);
+    else if (v4 && d4 <= 4096) LN4(1024, 4);
+    else hipLaunchKernelGGL(k_layernorm, dim3(rows), dim3(256), 0, s, x, g, b, d, eps, out, mean, rstd);
+#undef LN4
     LAUNCH_CHECK();
 }
 
@@ -284,7 +361,10 @@ int launch_rope_row(const float *x, size_t rows, int last_dim, int head_dim, con
 int launch_gather_cols(const float *x, size_t rows, int total, int start, int count, float *out, hipStream_t s) {
     const size_t n = rows * (size_t)count;
     if (n == 0) return SCRY_OK;
-    hipLaunchKernelGGL(k_gather_cols, dim3(grid1(n)), dim3(256), 0, s, x, rows, total, start, count, out);
+    if ((total | start | count) % 4 == 0)
+        hipLaunchKernelGGL(k_gather_cols<4>, dim3(grid1(n / 4)), dim3(256), 0, s, x, rows, total, start, count, out);
+    else
+        hipLaunchKernelGGL(k_gather_cols<1>, dim3(grid1(n)), dim3(256), 0, s, x, rows, total, start, count, out);
     LAUNCH_CHECK();
 }
 
@@ -330,16 +410,14 @@ int launch_add_inplace(float *d, const float *src, size_t n, hipStream_t s) {
     LAUNCH_CHECK();
 }
 
-int launch_scaled_softmax(const float *x, int rows, int cols, float scale, float *out, hipStream_t s) {
-    if (rows <= 0 || cols <= 0) return SCRY_OK;
-    hipLaunchKernelGGL(k_scaled_softmax, dim3(rows), dim3(256), 0, s, x, cols, scale, out);
-    LAUNCH_CHECK();
-}
-
 int launch_causal_mask(float *sc, size_t n_mat, int seq, float scale, float mask_value, hipStream_t s) {
-    const size_t n = n_mat * (size_t)seq * seq;
-    if (n == 0) return SCRY_OK;
-    hipLaunchKernelGGL(k_causal_mask, dim3(grid1(n)), dim3(256), 0, s, sc, n_mat, seq, scale, mask_value);
+    const size_t rows = n_mat * (size_t)seq;
+    if (rows == 0) return SCRY_OK;
+    const unsigned g = (unsigned)(rows < 65536 ? rows : 65536);
+    if (seq % 4 == 0)
+        hipLaunchKernelGGL(k_causal_mask<4>, dim3(g), dim3(256), 0, s, sc, rows, seq, scale, mask_value);
+    else
+        hipLaunchKernelGGL(k_causal_mask<1>, dim3(g), dim3(256), 0, s, sc, rows, seq, scale, mask_value);
     LAUNCH_CHECK();
 }
 
@@ -347,7 +425,10 @@ int launch_split_qkv(const float *qkv, int seq, int n_heads, int d_head, float *
                      hipStream_t s) {
     const size_t n = (size_t)seq * n_heads * d_head;
     if (n == 0) return SCRY_OK;
-    hipLaunchKernelGGL(k_split_qkv, dim3(grid1(n)), dim3(256), 0, s, qkv, seq, n_heads, d_head, q, k, v);
+    if (d_head % 4 == 0)
+        hipLaunchKernelGGL(k_split_qkv<4>, dim3(grid1(n / 4)), dim3(256), 0, s, qkv, seq, n_heads, d_head, q, k, v);
+    else
+        hipLaunchKernelGGL(k_split_qkv<1>, dim3(grid1(n)), dim3(256), 0, s, qkv, seq, n_heads, d_head, q, k, v);
     LAUNCH_CHECK();
 }
 
@@ -355,7 +436,12 @@ int launch_reshape_heads(const float *x, int batch, int seq, int n_heads, int d_
                          hipStream_t s) {
     const size_t n = (size_t)batch * seq * n_heads * d_head;
     if (n == 0) return SCRY_OK;
-    hipLaunchKernelGGL(k_reshape_heads, dim3(grid1(n)), dim3(256), 0, s, x, batch, seq, n_heads, d_head, dir, out);
+    if (d_head % 4 == 0)
+        hipLaunchKernelGGL(k_reshape_heads<4>, dim3(grid1(n / 4)), dim3(256), 0, s, x, batch, seq, n_heads, d_head, dir,
+                           out);
+    else
+        hipLaunchKernelGGL(k_reshape_heads<1>, dim3(grid1(n)), dim3(256), 0, s, x, batch, seq, n_heads, d_head, dir,
+                           out);
     LAUNCH_CHECK();
 }
 

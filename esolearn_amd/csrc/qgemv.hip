@@ -279,16 +279,6 @@ int launch_qgemv(int epi, const GemvArgs &g, hipStream_t s) {
     return set_error(SCRY_ERR_INVALID, "qgemv: unknown epilogue %d", epi);
 }
 
-// Ordered device argmax over one vector (generate.rs:167-173).
-namespace {
-__global__ __launch_bounds__(TPB) void k_argmax(const float *__restrict__ x, int n, int64_t *out) {
-    __shared__ ArgAcc sh[TPB];
-    ArgAcc r = block_argmax_range(x, 0, n, sh);
-    int tok = argmax_finish(r, x, n, sh);
-    if (threadIdx.x == 0) *out = (n <= 0) ? 0 : tok;
-}
-}  // namespace
-
 // End of a decode step: reduce the LM head's per-workgroup argmax partials in
 // index order (one workgroup), then record the token and advance the state.
 namespace {
@@ -336,13 +326,6 @@ int launch_logits_finish(const GemvArgs &g, hipStream_t s) {
     const int np = qgemv_blocks(EPI_LOGITS, *g.w, 1);
     hipLaunchKernelGGL(k_logits_finish, dim3(1), dim3(TPB), 0, s, g.y, g.w->rows, g.part_val,
                        g.part_idx, g.part_nan, np, g.state, g.tokens_rw, g.argmax_out, g.advance, g.ts);
-    SCRY_HIP(hipGetLastError());
-    return SCRY_OK;
-}
-
-int launch_argmax(const float *x, int64_t n, int64_t *out, hipStream_t s) {
-    if (n > 0x7fffffff) return set_error(SCRY_ERR_UNSUPPORTED, "argmax: n too large");
-    hipLaunchKernelGGL(k_argmax, dim3(1), dim3(TPB), 0, s, x, (int)n, out);
     SCRY_HIP(hipGetLastError());
     return SCRY_OK;
 }

@@ -74,16 +74,19 @@ struct SampleArgs {
     unsigned long long *rng;  // fastrand state
     DevState *st;
     int64_t *tokens;
-    // top-k off and V > LCAP: the statistics, exp values (ws) and 64-entry
-    // segment sums come from the two vocabulary-wide kernels below
+    // vocabulary-wide kernels before k_sample: the statistics (prep), and with
+    // top-k off and V > LCAP the exp values (ws) and 64-entry segment sums
+    // (segsum), with a small k the top-k candidates (cand, in ws)
     unsigned *prep;  // [PREP_WORDS], cleared by k_sample for the next step
-    double *segsum;  // [ceil(V / 64)]
+    double *segsum;  // [ceil(V / 64)] or null
+    const float2 *cand;  // (logit, index bits) or null
 };
 
 // prep words: the largest finite key, ~(smallest finite key), finite count,
 // NaN/+inf flag, ~(smallest key with e > 0) (atomic max of the complement:
 // all start at 0)
-enum { PR_MAXKEY = 0, PR_NKMIN = 1, PR_NFIN = 2, PR_BAD = 3, PR_NKMINP = 4, PREP_WORDS = 8 };
+// PR_NCAND: candidates written
+enum { PR_MAXKEY = 0, PR_NKMIN = 1, PR_NFIN = 2, PR_BAD = 3, PR_NKMINP = 4, PR_NCAND = 5, PREP_WORDS = 8 };
 
 __device__ __forceinline__ float key_f32(unsigned key) {  // inverse of okey
     return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
@@ -95,21 +98,8 @@ __device__ __forceinline__ bool draws(const DevState *st) {
     return p + 1 >= st->n_prompt && p + 1 <= st->max_tokens;
 }
 
-// Vocabulary-wide statistics for k_sample, over all CUs.
-__global__ __launch_bounds__(256) void k_prep_stats(const float *__restrict__ lg, int V, const DevState *st,
-                                                    unsigned *prep) {
-    if (!draws(st)) return;
-    unsigned kmax = 0, kmin = ~0u, nfin = 0, bad = 0;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < V; i += gridDim.x * 256) {
-        const float x = lg[i];
-        bad |= !(x < INFINITY);
-        if (x > -INFINITY && x < INFINITY) {
-            const unsigned k = okey(x);
-            kmax = max(kmax, k);
-            kmin = min(kmin, k);
-            nfin++;
-        }
-    }
+// one set of atomics per workgroup of 256 (they meet on four words in L2)
+__device__ __forceinline__ void stats_out(unsigned kmax, unsigned kmin, unsigned nfin, unsigned bad, unsigned *prep) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         kmax = max(kmax, (unsigned)__shfl_xor((int)kmax, off));
@@ -117,7 +107,6 @@ __global__ __launch_bounds__(256) void k_prep_stats(const float *__restrict__ lg
         nfin += (unsigned)__shfl_xor((int)nfin, off);
         bad |= (unsigned)__shfl_xor((int)bad, off);
     }
-    // one set of atomics per workgroup (they meet on four words in L2)
     __shared__ unsigned r[4][4];
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
@@ -139,6 +128,118 @@ __global__ __launch_bounds__(256) void k_prep_stats(const float *__restrict__ lg
         atomicAdd(prep + PR_NFIN, nfin);
         if (bad) atomicOr(prep + PR_BAD, 1u);
     }
+}
+
+// Vocabulary-wide statistics for k_sample, over all CUs.
+__global__ __launch_bounds__(256) void k_prep_stats(const float *__restrict__ lg, int V, const DevState *st,
+                                                    unsigned *prep) {
+    if (!draws(st)) return;
+    unsigned kmax = 0, kmin = ~0u, nfin = 0, bad = 0;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < V; i += gridDim.x * 256) {
+        const float x = lg[i];
+        bad |= !(x < INFINITY);
+        if (x > -INFINITY && x < INFINITY) {
+            const unsigned k = okey(x);
+            kmax = max(kmax, k);
+            kmin = min(kmin, k);
+            nfin++;
+        }
+    }
+    stats_out(kmax, kmin, nfin, bad, prep);
+}
+
+// Statistics and top-k candidates: every workgroup holds 2048 logits in
+// registers, finds its own k-th largest key (four 8-bit digits, histograms in
+// LDS) and appends its entries at or above it.  An entry at or above the
+// vocabulary's k-th largest has fewer than k larger ones anywhere, so it is
+// among its workgroup's: k_sample then selects among at most about k V / 2048
+// entries instead of passing over the vocabulary in one workgroup (V 128256,
+// k 40: 68 -> 24 us for both launches).
+constexpr int CAND_E = 8;         // entries per thread
+constexpr int CAND_MAXK = 256;    // GCAP: what finish_gather takes
+constexpr int CAND_MINV = 8192;   // below: one workgroup's passes are as fast
+__global__ __launch_bounds__(256) void k_prep_cand(const float *__restrict__ lg, int V, int k, const DevState *st,
+                                                   unsigned *prep, float2 *__restrict__ cand) {
+    if (!draws(st)) return;
+    __shared__ unsigned hist[256];
+    __shared__ unsigned wsum[4], s_bin, s_above, s_base;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float x[CAND_E];
+    unsigned key[CAND_E];
+    unsigned kmax = 0, kmin = ~0u, nfin = 0, bad = 0;
+#pragma unroll
+    for (int u = 0; u < CAND_E; u++) {
+        const int i = ((int)blockIdx.x * CAND_E + u) * 256 + tid;
+        x[u] = i < V ? lg[i] : -INFINITY;
+    }
+#pragma unroll
+    for (int u = 0; u < CAND_E; u++) {
+        bad |= !(x[u] < INFINITY);
+        const bool fin = x[u] > -INFINITY && x[u] < INFINITY;
+        key[u] = fin ? okey(x[u]) : 0u;  // 0: no finite key maps to it
+        if (fin) {
+            kmax = max(kmax, key[u]);
+            kmin = min(kmin, key[u]);
+            nfin++;
+        }
+    }
+    stats_out(kmax, kmin, nfin, bad, prep);
+    // the k-th largest key of this workgroup (0 when it holds fewer finite ones)
+    unsigned pre = 0, need = (unsigned)k;
+    for (int sh = 24; sh >= 0; sh -= 8) {
+        hist[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < CAND_E; u++)
+            if (key[u] && (sh == 24 || key[u] >> (sh + 8) == pre)) atomicAdd(&hist[(key[u] >> sh) & 255u], 1u);
+        __syncthreads();
+        // bins from the top: thread t holds bin 255 - t
+        const unsigned h = hist[255 - tid];
+        unsigned inc = h;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const unsigned o = (unsigned)__shfl_up((int)inc, off);
+            if (lane >= off) inc += o;
+        }
+        if (lane == 63) wsum[wave] = inc;
+        if (tid == 0) s_bin = ~0u;
+        __syncthreads();
+        for (int w = 0; w < wave; w++) inc += wsum[w];
+        if (inc - h < need && need <= inc) {
+            s_bin = 255u - (unsigned)tid;
+            s_above = inc - h;
+        }
+        __syncthreads();
+        if (s_bin == ~0u) {  // fewer than k finite entries (only at the first digit): all of them
+            pre = 0;
+            break;
+        }
+        need -= s_above;
+        pre = sh == 24 ? s_bin : (pre << 8) | s_bin;
+        __syncthreads();  // s_bin, hist are read above before the next digit writes them
+    }
+    unsigned n = 0;
+#pragma unroll
+    for (int u = 0; u < CAND_E; u++) n += key[u] && key[u] >= pre;
+    unsigned inc = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned o = (unsigned)__shfl_up((int)inc, off);
+        if (lane >= off) inc += o;
+    }
+    __syncthreads();  // wsum is read above
+    if (lane == 63) wsum[wave] = inc;
+    __syncthreads();
+    if (tid == 0) s_base = atomicAdd(prep + PR_NCAND, wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+    __syncthreads();
+    unsigned at = s_base + inc - n;
+    for (int w = 0; w < wave; w++) at += wsum[w];
+#pragma unroll
+    for (int u = 0; u < CAND_E; u++)
+        if (key[u] && key[u] >= pre) {
+            const int i = ((int)blockIdx.x * CAND_E + u) * 256 + tid;
+            cand[at++] = make_float2(x[u], __int_as_float(i));  // at < V: every entry at most once
+        }
 }
 
 // e = exp(f64(x)/f64(T) - max) for every entry (top-k off: every finite
@@ -263,6 +364,28 @@ struct Src {
     int V, nj;  // nj = ceil(V / SN) steps
 };
 
+// the candidate list visited like the vocabulary (each, with f's index the
+// entry's vocabulary index)
+struct CandSrc {
+    const float2 *c;
+    int n;
+};
+template <bool NE, class F>
+__device__ __forceinline__ void each(const CandSrc &s, F f) {
+    static_assert(!NE, "candidates carry no exp values");
+    for (int j0 = 0; j0 < s.n; j0 += 4 * SN) {
+        float2 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int j = j0 + u * SN + (int)threadIdx.x;
+            v[u] = j < s.n ? s.c[j] : make_float2(-INFINITY, 0.f);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            f(__float_as_int(v[u].y), v[u].x, 0.0, j0 + u * SN + (int)threadIdx.x < s.n);
+    }
+}
+
 // f(i, x, e, ok) for every step, all lanes of a wave together (f may vote);
 // ok = i < V; x = logits[i] (-inf past V); e = ws[i] when NE, else 0.
 template <bool NE, class F>
@@ -311,8 +434,8 @@ struct Sel {
 // the entry is a candidate.
 // With stop > 0 (UNIT only) it returns after the first level when the entries
 // at or above the chosen bin number at most stop.
-template <bool UNIT, class CW>
-__device__ __forceinline__ Sel select_top(const Src &src, unsigned kmin, unsigned kmax,
+template <bool UNIT, class SRC, class CW>
+__device__ __forceinline__ Sel select_top(const SRC &src, unsigned kmin, unsigned kmax,
                           unsigned long long T, CW cw, Shared &S, unsigned stop = 0) {
     const int tid = threadIdx.x;
     const unsigned span = kmax - kmin;
@@ -574,7 +697,8 @@ __device__ __forceinline__ int finish_small(const SampleArgs &a, const Src &src,
 // order, and the cumulative probability up to an index.
 constexpr int GCAP = SN / 4;
 
-__device__ __forceinline__ int finish_gather(const SampleArgs &a, const Src &src, Shared &S, unsigned lo,
+template <class SRC>
+__device__ __forceinline__ int finish_gather(const SampleArgs &a, const SRC &src, Shared &S, unsigned lo,
                                              unsigned k, double mxs, bool topp, unsigned long long Tp) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int V = a.V;
@@ -743,14 +867,18 @@ __device__ __forceinline__ int sample_body(const SampleArgs &a, Shared &S) {
     unsigned kk = kmin, nkept = nfin;
     const int k = a.top_k;
     if (k > 0 && k < V && nfin > (unsigned)k) {
-        const Sel s = select_top<true>(
-            src, kmin, kmax, (unsigned long long)k,
-            [&](float x, double, unsigned &key, unsigned long long &w) {
-                key = okey(x);
-                w = 1;
-                return x != -INFINITY;
-            },
-            S, GCAP);
+        auto finite = [&](float x, double, unsigned &key, unsigned long long &w) {
+            key = okey(x);
+            w = 1;
+            return x != -INFINITY;
+        };
+        if (a.cand) {  // every entry at or above the k-th key is a candidate
+            const CandSrc cs{a.cand, (int)a.prep[PR_NCAND]};
+            const Sel s = select_top<true>(cs, kmin, kmax, (unsigned long long)k, finite, S, GCAP);
+            if (s.small) return finish_gather(a, cs, S, s.lo, (unsigned)k, mxs, topp, Tp);
+            __syncthreads();  // (many equal logits: on to the vocabulary)
+        }
+        const Sel s = select_top<true>(src, kmin, kmax, (unsigned long long)k, finite, S, GCAP);
         if (s.small) return finish_gather(a, src, S, s.lo, (unsigned)k, mxs, topp, Tp);
         kk = s.key;
         nkept = (unsigned)(s.acc + s.nt);
@@ -761,7 +889,7 @@ __device__ __forceinline__ int sample_body(const SampleArgs &a, Shared &S) {
     // ---- 2. softmax over the kept entries
     double part = 0.0;
     unsigned kminp = ~0u;
-    if (a.prep) {  // exp values and segment sums from k_prep_exp
+    if (a.segsum) {  // exp values and segment sums from k_prep_exp
         for (int sg = tid; sg < nseg; sg += SN) part += a.segsum[sg];
         kminp = ~a.prep[PR_NKMINP];
     } else {
@@ -775,8 +903,8 @@ __device__ __forceinline__ int sample_body(const SampleArgs &a, Shared &S) {
         });
     }
     const double sum = block_sum(part, S.rd);
-    if (!a.prep) kminp = block_min_u(kminp, S.rk);
-    if (a.prep && !(a.top_p < 1.0f && a.top_p > 0.0f)) {
+    if (!a.segsum) kminp = block_min_u(kminp, S.rk);
+    if (a.segsum && !(a.top_p < 1.0f && a.top_p > 0.0f)) {
         // no top-p: r < sum(p up to i) is r * sum < sum(e up to i), up to rounding
         for (int sg = tid; sg < nseg; sg += SN) S.b.segq[sg] = a.segsum[sg];
         if (tid == 0) S.i0 = INT_MAX;
@@ -876,8 +1004,14 @@ __global__ __launch_bounds__(SN) void k_sample(SampleArgs a) {
 
 }  // namespace
 
+namespace {
+bool uses_cand(const scry_sampling_config &sc, int V) {
+    return sc.top_k > 0 && sc.top_k <= CAND_MAXK && V >= CAND_MINV;
+}
+}  // namespace
+
 bool sample_uses_prep(const scry_sampling_config &sc, int V) {
-    return (sc.top_k <= 0 || sc.top_k >= V) && V > LCAP;
+    return ((sc.top_k <= 0 || sc.top_k >= V) && V > LCAP) || uses_cand(sc, V);
 }
 
 size_t sample_prep_bytes(int V) { return sizeof(unsigned) * PREP_WORDS + sizeof(double) * ((V + 63) / 64); }
@@ -891,9 +1025,13 @@ int launch_sample(const float *logits, int V, const scry_sampling_config &sc, do
     const bool use = sample_uses_prep(sc, V);
     if (use && !prep) return set_error(SCRY_ERR_INVALID, "sample: missing the prep buffer");
     unsigned *pw = use ? (unsigned *)prep : nullptr;
-    double *seg = use ? (double *)((unsigned *)prep + PREP_WORDS) : nullptr;
-    SampleArgs a{logits, V, sc.temperature, sc.top_k, sc.top_p, ws, rng, st, tokens, pw, seg};
-    if (use) {
+    const bool cand = uses_cand(sc, V);
+    double *seg = use && !cand ? (double *)((unsigned *)prep + PREP_WORDS) : nullptr;
+    SampleArgs a{logits, V, sc.temperature, sc.top_k, sc.top_p, ws, rng, st, tokens, pw, seg, cand ? (const float2 *)ws : nullptr};
+    if (cand) {
+        hipLaunchKernelGGL(k_prep_cand, dim3((V + 256 * CAND_E - 1) / (256 * CAND_E)), dim3(256), 0, s, logits, V,
+                           sc.top_k, (const DevState *)st, pw, (float2 *)ws);
+    } else if (use) {
         const int nseg = (V + 63) / 64;
         hipLaunchKernelGGL(k_prep_stats, dim3(std::min(64, (V + 1023) / 1024)), dim3(256), 0, s, logits, V,
                            (const DevState *)st, pw);

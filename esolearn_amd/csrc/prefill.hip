@@ -688,14 +688,19 @@ __global__ __launch_bounds__(G_THREADS, B32 ? 1 : 2) void k_gemm(GemmP p) {
 // smaller tiles and k splits (pick_ring): with 128 x 256, 37 rows x 4096
 // columns are 16 workgroups.  Without splits a tile changes no bit (the k
 // order is the same); a split's f32 sums are added in split order.
-template <bool WBF, int BM_, int BN_, int WGM_, int WGN_, int S_>
+// B32: int8 weights with block-32 scales: the two scales a step has per column
+// ride in the stage, and a half step's products (one block) are scaled into
+// the sums.
+template <bool WBF, bool B32, int BM_, int BN_, int WGM_, int WGN_, int S_>
 struct RTile {
     static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, S = S_;
     static constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16, NW = WGM * WGN, T = 64 * NW;
     static constexpr int NPL = WBF ? 1 : 2, WB = WBF ? 2 : 1;  // activation planes; bytes per weight
-    static constexpr int A_PL = BM * BK * 2, B_ST = BN * BK * WB, STAGE = NPL * A_PL + B_ST;
+    static constexpr int A_PL = BM * BK * 2, B_ST = BN * BK * WB, SC = NPL * A_PL + B_ST;
+    static constexpr int STAGE = SC + (B32 ? 2 * BN * 4 : 0);  // scales [2][BN]
     static constexpr int JA = A_PL / 1024 / NW, JB = B_ST / 1024 / NW;  // 1 KB loads per wave and step
-    static constexpr int L = NPL * JA + JB;
+    static constexpr int L = NPL * JA + JB + (B32 ? 1 : 0);
+    static_assert(!B32 || (!WBF && 2 * (BN / 64) <= NW), "one 64-column scale load per wave");
     static constexpr size_t LDS = (size_t)S * STAGE;
     static constexpr bool BIG = BM_ == 128 && BN_ == 256;  // the super-tile map, no k splits
     static_assert(WGM * TM * 16 == BM && WGN * TN * 16 == BN && BK == 64, "ring tile");
@@ -703,8 +708,8 @@ struct RTile {
     static_assert(L * (S - 2) < 64, "vmcnt range");
     static_assert(LDS >= 2 * BM * (BN / 2 + 8) * sizeof(u16), "SwiGLU staging tile");
 };
-template <bool WBF>
-using RBig = RTile<WBF, BM, BN, 2, 4, 3>;
+template <bool WBF, bool B32>
+using RBig = RTile<WBF, B32, BM, BN, 2, 4, 3>;
 
 // buffer descriptor words (base, stride 0, num_records, raw-buffer flags),
 // wave-uniform
@@ -735,6 +740,19 @@ __device__ __forceinline__ void ring_load(u32x4 d, unsigned lds, unsigned voff, 
         : "s"(lds), "v"(voff), "s"(d), "s"(soff)
         : "memory");
 }
+// 64 lanes x 4 bytes of buffer d -> LDS [lds, lds + 256), as ring_load
+__device__ __forceinline__ void ring_load4(u32x4 d, unsigned lds, unsigned voff, unsigned soff) {
+    unsigned saved;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dword %2, %3, %4 offen lds\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(saved)
+        : "s"(lds), "v"(voff), "s"(d), "s"(soff)
+        : "memory");
+}
 template <int N>
 __device__ __forceinline__ void ring_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 // workgroup barrier without a memory fence (a fence would also wait for the
@@ -754,7 +772,7 @@ __device__ __forceinline__ bool small_tile(const GemmP &p, int &mb, int &nb, int
     return true;
 }
 
-template <int EPI, bool WBF, class C>
+template <int EPI, bool WBF, bool B32, class C>
 __global__ __launch_bounds__(C::T, C::BIG ? 1 : 2) void k_gemm_ring(GemmP p) {
     constexpr int A_PL = C::A_PL, STAGE = C::STAGE, JA = C::JA, L = C::L, NPL = C::NPL, WB = C::WB, S = C::S;
     constexpr int TM = C::TM, TN = C::TN, NW = C::NW, T = C::T, WGN = C::WGN;
@@ -770,13 +788,21 @@ __global__ __launch_bounds__(C::T, C::BIG ? 1 : 2) void k_gemm_ring(GemmP p) {
     const size_t a_bytes = (size_t)p.n_mb * C::BM * p.lda * 2;
     const u32x4 dh = ring_desc(p.ahi, a_bytes), dl = ring_desc(WBF ? p.ahi : p.alo, a_bytes);
     const u32x4 dw = ring_desc(p.w, (size_t)p.N * p.kp * WB);
+    const u32x4 dsc = ring_desc(B32 ? (const void *)p.s32 : p.w, B32 ? (size_t)p.N * p.nb * 4 : 4);
     const unsigned sm0 = (unsigned)(uintptr_t)sm;  // LDS address (low half of the flat address)
+    // B32: this wave's scale load fills block sc_h of 64 columns (waves past
+    // the last load the same again)
+    constexpr int SG = C::BN >= 64 ? C::BN / 64 : 1;
+    const int sc_u = wave % (2 * SG), sc_h = sc_u / SG;
+    const unsigned sc_lds = (unsigned)(C::SC + (sc_h * C::BN + (sc_u % SG) * 64) * 4);
+    const unsigned sc_voff = B32 ? (unsigned)(min(n0 + (sc_u % SG) * 64 + lane, p.N - 1) * p.nb * 4) : 0u;
     // load j of this wave fills 1 KB block u = j NW + wave: j < JA the hi plane
     // (8 rows of 128 B), j < 2 JA the lo plane, else the weights (int8: 16
     // columns of 64 B; bf16: 8 columns of 128 B)
-    unsigned voff[L], loff[L];
+    constexpr int LT = L - (B32 ? 1 : 0);  // loads of the tile
+    unsigned voff[LT], loff[LT];
 #pragma unroll
-    for (int j = 0; j < L; j++) {
+    for (int j = 0; j < LT; j++) {
         if (j < NPL * JA) {
             const int pl = j / JA, ua = (j % JA) * NW + wave;
             const int r = 8 * ua + (lane >> 3), c = (lane & 7) ^ (r & 7);
@@ -800,8 +826,9 @@ __global__ __launch_bounds__(C::T, C::BIG ? 1 : 2) void k_gemm_ring(GemmP p) {
     auto issue = [&](int kt, int slot) {
         const int ks = min(kt, kt1 - 1);
         const unsigned base = sm0 + (unsigned)(slot * STAGE);
+        if (B32) ring_load4(dsc, base + sc_lds, sc_voff, (unsigned)(min(2 * ks + sc_h, p.nb - 1) * 4));
 #pragma unroll
-        for (int j = 0; j < L; j++) {
+        for (int j = 0; j < LT; j++) {
             if (j < JA) ring_load(dh, base + loff[j], voff[j], (unsigned)(ks * BK * 2));
             else if (j < NPL * JA) ring_load(dl, base + loff[j], voff[j], (unsigned)(ks * BK * 2));
             else ring_load(dw, base + loff[j], voff[j], (unsigned)(ks * BK * WB));
@@ -831,6 +858,14 @@ __global__ __launch_bounds__(C::T, C::BIG ? 1 : 2) void k_gemm_ring(GemmP p) {
             if constexpr (WBF) {  // bf16 rows: chunk 2 g + h of the column's 128 bytes
                 b0[tn] = *(const bf16x8 *)(st + A_PL + n * 128 + (((2 * g) ^ (fr & 7)) << 4));
                 b1[tn] = *(const bf16x8 *)(st + A_PL + n * 128 + (((2 * g + 1) ^ (fr & 7)) << 4));
+            } else if constexpr (B32) {  // a half step is one block: 8 weights at k 32 h + 8 g
+                const int sw = (fr >> 1) & 3, lo8 = 8 * (g & 1);
+                const uint2 v0 = *(const uint2 *)(st + 2 * A_PL + n * 64 + (((g >> 1) ^ sw) << 4) + lo8);
+                const uint2 v1 = *(const uint2 *)(st + 2 * A_PL + n * 64 + (((2 + (g >> 1)) ^ sw) << 4) + lo8);
+                u32x4 o0, o1;
+                bytes_to_bf16(u32x4{v0.x, v0.y, v1.x, v1.y}, o0, o1);
+                b0[tn] = __builtin_bit_cast(bf16x8, o0);
+                b1[tn] = __builtin_bit_cast(bf16x8, o1);
             } else {
                 const u32x4 v = *(const u32x4 *)(st + 2 * A_PL + n * 64 + ((g ^ ((fr >> 1) & 3)) << 4));
                 u32x4 o0, o1;
@@ -844,9 +879,28 @@ __global__ __launch_bounds__(C::T, C::BIG ? 1 : 2) void k_gemm_ring(GemmP p) {
             bf16x8 ah[TM], al[TM];
 #pragma unroll
             for (int tm = 0; tm < TM; tm++) {
-                const int off = (wm * TM * 16 + tm * 16 + fr) * 128 + (((2 * g + h) ^ (fr & 7)) << 4);
+                const int ch = B32 ? 4 * h + g : 2 * g + h;  // 16-byte chunk of the row's 128
+                const int off = (wm * TM * 16 + tm * 16 + fr) * 128 + ((ch ^ (fr & 7)) << 4);
                 ah[tm] = *(const bf16x8 *)(st + off);
                 if (!WBF) al[tm] = *(const bf16x8 *)(st + A_PL + off);
+            }
+            if constexpr (B32) {
+#pragma unroll
+                for (int tn = 0; tn < TN; tn++) {
+                    const float sc = *(const float *)(st + C::SC + (h * C::BN + wn * TN * 16 + tn * 16 + fr) * 4);
+                    f32x4 t[TM];
+#pragma unroll
+                    for (int tm = 0; tm < TM; tm++)
+                        t[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[tm], h ? b1[tn] : b0[tn], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                    for (int tm = 0; tm < TM; tm++)
+                        t[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[tm], h ? b1[tn] : b0[tn], t[tm], 0, 0, 0);
+#pragma unroll
+                    for (int tm = 0; tm < TM; tm++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) acc[tm][tn][r] = fmaf(sc, t[tm][r], acc[tm][tn][r]);
+                }
+                continue;
             }
 #pragma unroll
             for (int tn = 0; tn < TN; tn++)
@@ -880,7 +934,7 @@ __global__ __launch_bounds__(C::T, C::BIG ? 1 : 2) void k_gemm_ring(GemmP p) {
     }
     if (EPI == GE_SWIGLU) {
         __syncthreads();  // every wave's tail loads have landed
-        swiglu_store<TM, TN, T, WBF, C::BM, C::BN>(p, acc, reinterpret_cast<u16 *>(sm), wm * TM * 16, wn * TN * 16, m0,
+        swiglu_store<TM, TN, T, WBF || B32, C::BM, C::BN>(p, acc, reinterpret_cast<u16 *>(sm), wm * TM * 16, wn * TN * 16, m0,
                                                    n0, lane);
         if (wave == 0 && nbk == p.n_nb - 1) swiglu_pad<C::BM>(p, m0, lane);
     } else {
@@ -1727,12 +1781,16 @@ int digits_small(GemmP p, int splits, hipStream_t s) {
 //   bf16    512 x 11008 x 4096 180 -> 65, 37 x 4096 x 12288 63 -> 22, 37 x
 //           11008 x 4096 152 -> 22, 130 x 4096 x 28672 134 -> 81, 256 x 768 x
 //           2304 22 -> 8; kept: 512 x 4096 x 28672 157 (next best 188)
+//   block-32, against the register-staged kernel: 37 x 4096 x 14336 251 -> 38,
+//           130 x 11008 x 4096 661 -> 75, 512 x 11008 x 4096 673 -> 144, 1024 x
+//           4096 x 14336 523 -> 315 (large tile)
 struct TileCost {
     int bm, bn;
     double alone, shared;
 };
 constexpr TileCost kDigitTiles[5] = {{128, 256, 1.25, 1.25}, {128, 128, 0.80, 0.80}, {64, 128, 0.52, 0.50}, {64, 64, 0.38, 0.345}, {32, 128, 0.376, 0.34}};
 constexpr TileCost kRingTiles[5] = {{128, 256, 1.15, 1.20}, {128, 128, 0.65, 0.70}, {64, 128, 0.42, 0.36}, {64, 64, 0.33, 0.23}, {32, 128, 0.34, 0.26}};
+constexpr TileCost kB32Tiles[5] = {{128, 256, 2.2, 2.4}, {128, 128, 1.42, 1.38}, {64, 128, 0.92, 0.74}, {64, 64, 0.62, 0.49}, {32, 128, 0.60, 0.52}};
 struct TilePick {
     int tile, splits;
 };
@@ -1766,19 +1824,19 @@ int gemm_digits_t(const GemmP &p, hipStream_t s) {
     return digits_launch<EPI, DBig>(p, (p.n_super + 7) / 8 * 8 * 32, s);
 }
 
-template <int EPI, bool WBF, class C>
+template <int EPI, bool WBF, bool B32, class C>
 int ring_launch(const GemmP &p, int grid, hipStream_t s) {
     static bool attr = false;
     if (!attr) {
-        SCRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gemm_ring<EPI, WBF, C>),
+        SCRY_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gemm_ring<EPI, WBF, B32, C>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS));
         attr = true;
     }
-    hipLaunchKernelGGL((k_gemm_ring<EPI, WBF, C>), dim3(grid), dim3(C::T), C::LDS, s, p);
+    hipLaunchKernelGGL((k_gemm_ring<EPI, WBF, B32, C>), dim3(grid), dim3(C::T), C::LDS, s, p);
     PF_LAUNCH_CHECK();
 }
 
-template <int EPI, class C>
+template <int EPI, bool WBF, bool B32, class C>
 int ring_small(GemmP p, int splits, hipStream_t s) {
     p.n_mb = (p.M + C::BM - 1) / C::BM;
     p.n_nb = (p.N + C::BN - 1) / C::BN;
@@ -1789,7 +1847,7 @@ int ring_small(GemmP p, int splits, hipStream_t s) {
         SCRY_TRY(ctx_workspace(sizeof(float) * (size_t)p.splits * p.M * p.N, &ws));
         p.partf = (float *)ws;
     }
-    SCRY_TRY((ring_launch<EPI, true, C>(p, (p.n_mb * p.n_nb * p.splits + 7) / 8 * 8, s)));
+    SCRY_TRY((ring_launch<EPI, WBF, B32, C>(p, (p.n_mb * p.n_nb * p.splits + 7) / 8 * 8, s)));
     if (p.splits > 1) {
         const size_t g = ((size_t)p.M * p.N + 255) / 256;
         hipLaunchKernelGGL(k_ring_finish<EPI>, dim3((unsigned)std::min<size_t>(g, 65536)), dim3(256), 0, s, p);
@@ -1798,19 +1856,21 @@ int ring_small(GemmP p, int splits, hipStream_t s) {
     return SCRY_OK;
 }
 
-template <int EPI, bool WBF>
+// WBF or B32: the tile by pick_tile; int8 per-tensor weights through bf16
+// planes (k beyond the digit kernel's): the large tile
+template <int EPI, bool WBF, bool B32 = false>
 int gemm_ring_t(const GemmP &p, hipStream_t s) {
-    if constexpr (WBF) {
+    if constexpr (WBF || B32) {
         // SwiGLU planes come from the whole sums: no k splits
-        const TilePick d = pick_tile(kRingTiles, p.M, p.N, p.nk, sizeof(float), 5, EPI == GE_SWIGLU ? 1 : 8);
+        const TilePick d = pick_tile(B32 ? kB32Tiles : kRingTiles, p.M, p.N, p.nk, sizeof(float), 5, EPI == GE_SWIGLU ? 1 : 8);
         switch (d.tile) {
-            case 1: return ring_small<EPI, RTile<true, 128, 128, 2, 4, 3>>(p, d.splits, s);
-            case 2: return ring_small<EPI, RTile<true, 64, 128, 2, 2, 3>>(p, d.splits, s);
-            case 3: return ring_small<EPI, RTile<true, 64, 64, 2, 2, 4>>(p, d.splits, s);
-            case 4: return ring_small<EPI, RTile<true, 32, 128, 1, 4, 4>>(p, d.splits, s);
+            case 1: return ring_small<EPI, WBF, B32, RTile<WBF, B32, 128, 128, 2, 4, 3>>(p, d.splits, s);
+            case 2: return ring_small<EPI, WBF, B32, RTile<WBF, B32, 64, 128, 2, 2, 3>>(p, d.splits, s);
+            case 3: return ring_small<EPI, WBF, B32, RTile<WBF, B32, 64, 64, 2, 2, B32 ? 3 : 4>>(p, d.splits, s);
+            case 4: return ring_small<EPI, WBF, B32, RTile<WBF, B32, 32, 128, 1, 4, 4>>(p, d.splits, s);
         }
     }
-    return ring_launch<EPI, WBF, RBig<WBF>>(p, (p.n_super + 7) / 8 * 8 * 32, s);
+    return ring_launch<EPI, WBF, B32, RBig<WBF, B32>>(p, (p.n_super + 7) / 8 * 8 * 32, s);
 }
 
 }  // namespace
@@ -1956,10 +2016,12 @@ int launch_gemm(int epi, const PrefillGemm &g, hipStream_t s) {
         return set_error(SCRY_ERR_INVALID, "gemm: unknown epilogue %d", epi);
     }
     if (b32) {
+        p.scale = p.scale2 = 1.f;  // the block scales are in the sums
+        const bool r = ring_ok && (size_t)p.N * p.nb * 4 < 0x7fffffffull;
         switch (epi) {
-            case GE_STORE: return gemm_t<GE_STORE, true>(p, s);
-            case GE_RESID: return gemm_t<GE_RESID, true>(p, s);
-            case GE_SWIGLU: return gemm_t<GE_SWIGLU, true>(p, s);
+            case GE_STORE: return r ? gemm_ring_t<GE_STORE, false, true>(p, s) : gemm_t<GE_STORE, true>(p, s);
+            case GE_RESID: return r ? gemm_ring_t<GE_RESID, false, true>(p, s) : gemm_t<GE_RESID, true>(p, s);
+            case GE_SWIGLU: return r ? gemm_ring_t<GE_SWIGLU, false, true>(p, s) : gemm_t<GE_SWIGLU, true>(p, s);
         }
         return set_error(SCRY_ERR_INVALID, "gemm: unknown epilogue %d", epi);
     }

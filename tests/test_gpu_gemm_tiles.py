@@ -93,3 +93,36 @@ def test_bf16_prefill_small_tiles_match_decode(hip, seq):
         ref, _ = m.forward_with_llama_cache(int(t), p, cd)
     assert np.abs(last - ref).max() <= 1e-2 * np.abs(ref).max()
     m.free()
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (17, 64, 5), (33, 100, 131), (40, 4096, 260), (64, 768, 768), (130, 3000, 1030), (129, 4096, 4096),
+    (300, 1024, 4097), (512, 11008, 516)])
+def test_block32_exact_sums(hip, m, k, n):
+    """Block-32 scales that are powers of two: every product and sum is exact in f32."""
+    print(f"[case] block32 {m} x {k} x {n}", flush=True)
+    B = hip.HipBackend
+    rng = np.random.default_rng(m + k + n)
+    nb = (k + 31) // 32
+    a = rng.integers(-3, 4, (m, k)).astype(F)
+    q = rng.integers(-40, 41, (k, n)).astype(np.int8)
+    s = (2.0 ** rng.integers(-2, 2, (n, nb))).astype(F)
+    w = q * s.repeat(32, axis=1)[:, :k].T.astype(np.float64)
+    c = B.matmul_i8_f32_block32(B.from_vec(a), B.i8_from_vec(q), B.from_vec(s), m, k, n).to_vec().reshape(m, n)
+    assert np.array_equal(c, a.astype(np.float64) @ w)
+
+
+@pytest.mark.parametrize("seq", [18, 130])
+def test_block32_prefill_matches_decode(hip, seq):
+    print(f"[case] block32 seq={seq}", flush=True)
+    import esolearn_amd.llama as EL
+    cfg = hip.LlamaConfig(vocab_size=96, hidden_size=2048, intermediate_size=4100, n_layers=1, n_heads=16,
+                          n_kv_heads=4, max_seq_len=256, rope_theta=10000.0, tie_word_embeddings=False)
+    m = hip.LlamaModel.new_random(cfg, 3, quant_mode=EL.QUANT_BLOCK32, init_on_device=True)
+    toks = np.random.default_rng(seq).integers(0, 96, seq)
+    cp, cd = m.new_llama_kv_cache(seq), m.new_llama_kv_cache(seq)
+    last = m.prefill([cp], toks[None, :])[0]
+    for p, t in enumerate(toks):
+        ref, _ = m.forward_with_llama_cache(int(t), p, cd)
+    assert np.abs(last - ref).max() <= 1e-3 * np.abs(ref).max()
+    m.free()

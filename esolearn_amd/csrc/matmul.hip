@@ -38,8 +38,8 @@ struct MMArgs {
 // requested before the current step's MFMAs and written to the other LDS
 // buffer after them (one barrier per step).
 // Measured against one thread per output with a serial f64 loop: 1500 x 1280
-// x 5120 (k in the middle) 385 us, 51 TFLOP/s, against about 10 ms; attention
-// scores 20 x [1500 x 64] x [64 x 1500] 146 us against 2.7 ms, values 130 us.
+// x 5120 (k in the middle) 368 us, 53 TFLOP/s, against about 10 ms; attention
+// scores 20 x [1500 x 64] x [64 x 1500] 134 us against 2.7 ms, values 123 us.
 constexpr int MM_T = 256, MM_BK = 32, MM_S = 36;
 
 // KC: the operand is stored k-contiguous ([row][k], ld = k), else [k][row]
@@ -132,8 +132,12 @@ struct Stage {
     }
 };
 
+// Two waves per SIMD at least: with at most 256 registers the compiler keeps
+// the sums in vector registers; otherwise it moved all of them to accumulation
+// registers and back in every step (64 moves per 32 MFMAs: 1500 x 1280 x 5120
+// 385 us, now 368; attention scores 146 -> 134, values 130 -> 123).
 template <int BM, int BN, bool TA, bool TB, int LD>
-__global__ __launch_bounds__(MM_T) void k_mm_f64(MMArgs p) {
+__global__ __launch_bounds__(MM_T, 2) void k_mm_f64(MMArgs p) {
     __shared__ __align__(16) float sa[2][BM * MM_S];
     __shared__ __align__(16) float sb[2][BN * MM_S];
     constexpr int WM = BM / 2, WN = BN / 2, NM = WM / 16, NN = WN / 16;
@@ -194,12 +198,6 @@ __global__ __launch_bounds__(MM_T) void k_mm_f64(MMArgs p) {
         }
         la.store(sa[cur ^ 1]);
         lb.store(sb[cur ^ 1]);
-        // the sums stay in accumulation registers across steps (without this
-        // the compiler moves all of them to vector registers and back)
-#pragma unroll
-        for (int x = 0; x < NM; x++)
-#pragma unroll
-            for (int y = 0; y < NN; y++) asm volatile("" : "+a"(acc[x][y]));
         __syncthreads();
         cur ^= 1;
     }
@@ -471,9 +469,9 @@ int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, i
     auto tiles = [&](int t) { return (size_t)batch * ((m + t - 1) / t) * ((n + t - 1) / t); };
     const bool wide = std::max({m, n, k}) > (1 << 21);  // 31-bit offsets: 128 rows of k, or 32 k rows of m or n values
     // 64 x 64 tiles where they fill the CUs or a long k can be split over
-    // them, else 32 x 32 (12 x 200 x 200 x 64: 7 against 14 us; 64 x 4096 x
-    // 4096, split: 62 against 53 us).  128 x 128 was slower everywhere
-    // (1500 x 1280 x 5120: 513 against 385 us, one wave per SIMD).
+    // them, else 32 x 32 (12 x 200 x 200 x 64: 6 against 14 us; 64 x 4096 x
+    // 4096, split: 62 against 49 us).  128 x 128 was slower everywhere
+    // (1500 x 1280 x 5120: 513 against 368 us, one wave per SIMD).
     const int steps = (k + MM_BK - 1) / MM_BK;
     const int t = tiles(64) >= 256 || (steps >= 64 && m > 32 && n > 32) ? 64 : 32;
     p.tm = (m + t - 1) / t;

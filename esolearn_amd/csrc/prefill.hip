@@ -283,7 +283,6 @@ struct GemmP {
     int nb;
     int M, nk;         // rows, k steps (k rounded up to 32, / 32)
     int n_mb, n_nb;    // tiles along M and N
-    int n_super;       // super-tiles (4 M tiles x 8 N tiles)
     float scale, scale2;
     const float *bias;  // GE_STORE: + bias[n] (f32, after scaling)
     float *c;
@@ -299,19 +298,25 @@ struct GemmP {
     float *partf;           // the same for k_gemm_ring
 };
 
-// Workgroup -> tile: workgroup b runs on XCD b % 8.  Tiles are grouped in
-// super-tiles of 4 M tiles x 8 N tiles; an XCD works through whole
-// super-tiles, so the workgroups it runs together share A rows and weight
-// rows in its L2.
+// Workgroup -> tile: workgroup b runs on XCD b % 8.  Tiles are numbered by
+// super-tiles of 4 M tiles x 8 N tiles (fewer at the last rows and columns) and
+// an XCD works through whole runs of 32 of them, so the workgroups it runs
+// together share A rows and weight rows in its L2.  Only real tiles are
+// numbered: with 32 numbers for every super-tile, 2 row tiles x 112 column
+// tiles took two rounds of the chip instead of one (130 x 4096 x 28672 150 ->
+// 83 us, 640 x 4096 x 28672 300 -> 231).
 __device__ __forceinline__ bool gemm_tile(const GemmP &p, int &mb, int &nb) {
     const int b = blockIdx.x, xcd = b & 7, loc = b >> 3;
-    const int sup = (loc >> 5) * 8 + xcd, in = loc & 31;
-    if (sup >= p.n_super) return false;
-    const int n_msup = (p.n_mb + 3) >> 2;
-    mb = (sup % n_msup) * 4 + (in & 3);
-    nb = (sup / n_msup) * 8 + (in >> 2);
-    return mb < p.n_mb && nb < p.n_nb;
+    const int t = ((loc >> 5) * 8 + xcd) * 32 + (loc & 31);
+    if (t >= p.n_mb * p.n_nb) return false;
+    const int nb0 = t / (8 * p.n_mb) * 8, nw = min(8, p.n_nb - nb0);  // panel of column tiles
+    const int in = t - nb0 * p.n_mb, mb0 = in / (4 * nw) * 4, mh = min(4, p.n_mb - mb0);
+    const int r = in - mb0 * nw;
+    mb = mb0 + r % mh;
+    nb = nb0 + r / mh;
+    return true;
 }
+int gemm_tile_grid(const GemmP &p) { return (p.n_mb * p.n_nb + 255) / 256 * 256; }
 
 // 16 weight bytes (q + 128) -> 16 bf16 of q, as 8 words.  Flipping bit 7
 // gives q's two's-complement byte; |q| <= 128 is exact in bf16
@@ -1732,8 +1737,7 @@ int gemm_t(const GemmP &p, hipStream_t s) {
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMM_LDS));
         attr = true;
     }
-    const int grid = (p.n_super + 7) / 8 * 8 * 32;
-    hipLaunchKernelGGL((k_gemm<EPI, B32, WBF>), dim3(grid), dim3(G_THREADS), GEMM_LDS, s, p);
+    hipLaunchKernelGGL((k_gemm<EPI, B32, WBF>), dim3(gemm_tile_grid(p)), dim3(G_THREADS), GEMM_LDS, s, p);
     PF_LAUNCH_CHECK();
 }
 
@@ -1821,7 +1825,7 @@ int gemm_digits_t(const GemmP &p, hipStream_t s) {
         case 3: return digits_small<EPI, DTile<64, 64, 2, 2, 4>>(p, d.splits, s);
         case 4: return digits_small<EPI, DTile<32, 128, 1, 2, 4>>(p, d.splits, s);
     }
-    return digits_launch<EPI, DBig>(p, (p.n_super + 7) / 8 * 8 * 32, s);
+    return digits_launch<EPI, DBig>(p, gemm_tile_grid(p), s);
 }
 
 template <int EPI, bool WBF, bool B32, class C>
@@ -1870,7 +1874,7 @@ int gemm_ring_t(const GemmP &p, hipStream_t s) {
             case 4: return ring_small<EPI, WBF, B32, RTile<WBF, B32, 32, 128, 1, 4, 4>>(p, d.splits, s);
         }
     }
-    return ring_launch<EPI, WBF, B32, RBig<WBF, B32>>(p, (p.n_super + 7) / 8 * 8 * 32, s);
+    return ring_launch<EPI, WBF, B32, RBig<WBF, B32>>(p, gemm_tile_grid(p), s);
 }
 
 }  // namespace
@@ -1984,7 +1988,6 @@ int launch_gemm(int epi, const PrefillGemm &g, hipStream_t s) {
     p.nk = kpad / BK;
     p.n_mb = (g.M + BM - 1) / BM;
     p.n_nb = (w.rows + BN - 1) / BN;
-    p.n_super = ((p.n_mb + 3) / 4) * ((p.n_nb + 7) / 8);
     p.scale = w.scale;
     p.scale2 = w.scale2;
     p.bias = g.bias;
@@ -2059,7 +2062,6 @@ int launch_gemm_bf16(const unsigned short *w, int kp, int N, int k, const unsign
     p.nk = kpad / BK;
     p.n_mb = (M + BM - 1) / BM;
     p.n_nb = (N + BN - 1) / BN;
-    p.n_super = ((p.n_mb + 3) / 4) * ((p.n_nb + 7) / 8);
     p.scale = 1.f;
     p.scale2 = 1.f;
     p.bias = bias;

@@ -11,7 +11,8 @@ F = np.float32
 
 @pytest.mark.parametrize("m,k,n", [
     (17, 64, 5), (33, 100, 131), (32, 2048, 128), (37, 4096, 260), (64, 768, 768), (65, 3072, 770),
-    (130, 4096, 1030), (200, 768, 2304), (129, 8192, 4096), (300, 1024, 4097), (512, 2048, 2050)])
+    (130, 4096, 1030), (200, 768, 2304), (129, 8192, 4096), (300, 1024, 4097), (512, 2048, 2050),
+    (129, 256, 28416), (600, 128, 28000), (255, 192, 21889), (1100, 64, 13000)])
 def test_exact_sums(hip, m, k, n):
     print(f"[case] {m} x {k} x {n}", flush=True)
     B = hip.HipBackend

@@ -989,11 +989,12 @@ struct DTile {
     static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, S = S_;
     static constexpr int TM = BM / WGM / 16, TN = BN / WGN / 16, NW = WGM * WGN, T = 64 * NW;
     static constexpr int A_PL = BM * BK, B_ST = BN * BK, STAGE = 3 * A_PL + B_ST;
-    static constexpr int JP = 3 * A_PL / 1024 / NW, JB = B_ST / 1024 / NW, L = JP + JB;  // 1 KB loads (16 rows of 64 B)
+    // 1 KB loads per wave (16 rows of 64 B); weight loads past the last unit repeat it
+    static constexpr int JP = 3 * A_PL / 1024 / NW, BU = B_ST / 1024, JB = (BU + NW - 1) / NW, L = JP + JB;
     static constexpr size_t LDS = (size_t)S * STAGE;
     static constexpr bool BIG = BM_ == 128 && BN_ == 256;  // k_gemm_ring's tile and map
     static_assert(BK == 64 && WGM * TM * 16 == BM && WGN * TN * 16 == BN, "digit ring tile");
-    static_assert(3 * A_PL / 1024 % NW == 0 && B_ST / 1024 % NW == 0, "digit ring units");
+    static_assert(3 * A_PL / 1024 % NW == 0, "digit ring units");
     static_assert(L * (S - 2) < 64, "vmcnt range");
     static_assert(LDS >= BM * (BN / 2 + 4) * sizeof(float), "SwiGLU staging tile");
 };
@@ -1032,7 +1033,7 @@ __global__ __launch_bounds__(TL::T, TL::BIG ? 1 : 2) void k_gemm_digits(GemmP p)
             voff[j] = (unsigned)(pl * p.dstride + (size_t)(m0 + r) * p.lda + c * 16);
             loff[j] = (unsigned)(pl * A_PL + ua * 1024);
         } else {
-            const int ub = (j - JP) * NW + wave;
+            const int ub = min((j - JP) * NW + wave, TL::BU - 1);
             const int n = 16 * ub + (lane >> 2), c = (lane & 3) ^ ((n >> 1) & 3);
             const int row = min(n0 + n, p.N - 1);  // columns past N re-read row N - 1 (never stored)
             voff[j] = (unsigned)(row * p.kp + c * 16);
@@ -1781,7 +1782,10 @@ int digits_small(GemmP p, int splits, hipStream_t s) {
 // the fastest.  Measured, that tile -> this choice (rows x k x n):
 //   digits  512 x 11008 x 4096 193 -> 91 us, 512 x 4096 x 4096 81 -> 43, 130 x
 //           4096 x 14336 80 -> 57, 64 x 11008 x 4096 180 -> 29, 200 x 768 x
-//           2304 26 -> 11; kept: 512 x 4096 x 14336 89 (next best 113)
+//           2304 26 -> 11; kept: 512 x 4096 x 14336 89 (next best 113).  128 x
+//           192 where the others leave the last round part empty: 130 x 4096 x
+//           22016 82 -> 74, 1024 x 4096 x 6144 87 -> 81; not 1024 x 4096 x
+//           14336 (167, it 220)
 //   bf16    512 x 11008 x 4096 180 -> 65, 37 x 4096 x 12288 63 -> 22, 37 x
 //           11008 x 4096 152 -> 22, 130 x 4096 x 28672 134 -> 81, 256 x 768 x
 //           2304 22 -> 8; kept: 512 x 4096 x 28672 157 (next best 188)
@@ -1792,15 +1796,15 @@ struct TileCost {
     int bm, bn;
     double alone, shared;
 };
-constexpr TileCost kDigitTiles[5] = {{128, 256, 1.25, 1.25}, {128, 128, 0.80, 0.80}, {64, 128, 0.52, 0.50}, {64, 64, 0.38, 0.345}, {32, 128, 0.376, 0.34}};
+constexpr TileCost kDigitTiles[6] = {{128, 256, 1.25, 1.25}, {128, 128, 0.80, 0.80}, {64, 128, 0.52, 0.50}, {64, 64, 0.38, 0.345}, {32, 128, 0.376, 0.34}, {128, 192, 1.12, 1.14}};
 constexpr TileCost kRingTiles[5] = {{128, 256, 1.15, 1.20}, {128, 128, 0.65, 0.70}, {64, 128, 0.42, 0.36}, {64, 64, 0.33, 0.23}, {32, 128, 0.34, 0.26}};
 constexpr TileCost kB32Tiles[5] = {{128, 256, 2.2, 2.4}, {128, 128, 1.42, 1.38}, {64, 128, 0.92, 0.74}, {64, 64, 0.62, 0.49}, {32, 128, 0.60, 0.52}};
 struct TilePick {
     int tile, splits;
+    double t;
 };
-TilePick pick_tile(const TileCost (&tl)[5], int M, int N, int nk, int part_bytes, int n_tiles, int max_splits) {
-    TilePick best{0, 1};
-    double bt = 1e30;
+TilePick pick_tile(const TileCost *tl, int n_tiles, int M, int N, int nk, int part_bytes, int max_splits) {
+    TilePick best{0, 1, 1e30};
     for (int i = 0; i < n_tiles; i++) {
         const double tiles = (double)((M + tl[i].bm - 1) / tl[i].bm) * ((N + tl[i].bn - 1) / tl[i].bn);
         for (int sp = 1; sp <= (i ? max_splits : 1); sp *= 2) {
@@ -1809,23 +1813,76 @@ TilePick pick_tile(const TileCost (&tl)[5], int M, int N, int nk, int part_bytes
             const double n = std::ceil(tiles * sp / 256.0);
             double t = (nk + sp - 1) / sp * n * (n > 1 ? tl[i].shared : tl[i].alone);
             if (sp > 1) t += 4.0 + 2.0 * bytes / 5.0e6;
-            if (t < bt) bt = t, best = {i, sp};
+            if (t < best.t) best = {i, sp, t};
         }
     }
     return best;
 }
 
+// A last round of the chip that is mostly empty costs a whole one.  Where it is
+// 4 % cheaper (below that the model cannot tell: 1500 x 11008 x 4096 was 5 %
+// slower at 1 %), the columns of the full rounds go to one launch and the rest
+// to a second one with its own tile, 6 us allowed for launch and drain.
+// Measured, one launch of the best tile -> two:
+//   digits    384 x 4096 x 22016 147 -> 103 us, 511 x 4096 x 22016 149 -> 139,
+//             600 x 4096 x 14336 146 -> 123, 1500 x 4096 x 22016 377 -> 339
+//   block-32  384 x 4096 x 22016 238 -> 177, 600 x 4096 x 14336 244 -> 198,
+//             2046 x 4096 x 14336 605 -> 546
+struct CutPick {
+    TilePick first, rest;
+    int cols;  // columns of the first launch; 0 = one launch (first)
+};
+CutPick pick_cut(const TileCost *tl, int n_tiles, int M, int N, int nk, int part_bytes, int max_splits) {
+    CutPick best{pick_tile(tl, n_tiles, M, N, nk, part_bytes, max_splits), {}, 0};
+    double bt = 0.96 * best.first.t;
+    for (int i = 0; i < n_tiles; i++) {
+        const int n_mb = (M + tl[i].bm - 1) / tl[i].bm, n_nb = (N + tl[i].bn - 1) / tl[i].bn;
+        const int rounds = (int)((int64_t)n_mb * n_nb / 256);
+        const int64_t cols = (int64_t)rounds * 256 / n_mb * tl[i].bn;
+        if (cols < 1 || cols >= N) continue;
+        const TilePick r = pick_tile(tl, n_tiles, M, N - (int)cols, nk, part_bytes, max_splits);
+        const double t = nk * rounds * (rounds > 1 ? tl[i].shared : tl[i].alone) + 6.0 + r.t;
+        if (t < bt) bt = t, best = {{i, 1, 0.0}, r, (int)cols};
+    }
+    return best;
+}
+
+// columns [c0, c0 + n) of p as a problem of their own (c0 a multiple of 64;
+// el: bytes of a weight)
+GemmP gemm_cols(GemmP p, int c0, int n, int el) {
+    const bool end = c0 + n == p.N;
+    p.w += (size_t)c0 * p.kp * el;
+    if (p.s32) p.s32 += (size_t)c0 * p.nb;
+    if (p.bias) p.bias += c0;
+    if (p.c) p.c += c0;
+    if (p.of) p.of += c0 / 2;  // the SwiGLU outputs: one column per two
+    if (p.ohi) p.ohi += c0 / 2;
+    if (p.olo) p.olo += c0 / 2;
+    p.opad = end ? p.opad - c0 / 2 : n / 2;  // the zero pad comes with the last columns
+    p.N = n;
+    p.n_nb = (n + BN - 1) / BN;
+    return p;
+}
+
 template <int EPI>
-int gemm_digits_t(const GemmP &p, hipStream_t s) {
-    // the smaller tiles write SwiGLU as f32 rows only
-    const TilePick d = pick_tile(kDigitTiles, p.M, p.N, p.nk, sizeof(double), EPI != GE_SWIGLU || p.of ? 5 : 1, 16);
+int gemm_digits_tile(const GemmP &p, const TilePick &d, hipStream_t s) {
     switch (d.tile) {
         case 1: return digits_small<EPI, DTile<128, 128, 2, 4, 3>>(p, d.splits, s);
         case 2: return digits_small<EPI, DTile<64, 128, 2, 2, 3>>(p, d.splits, s);
         case 3: return digits_small<EPI, DTile<64, 64, 2, 2, 4>>(p, d.splits, s);
         case 4: return digits_small<EPI, DTile<32, 128, 1, 2, 4>>(p, d.splits, s);
+        case 5: return digits_small<EPI, DTile<128, 192, 2, 4, 3>>(p, d.splits, s);
     }
     return digits_launch<EPI, DBig>(p, gemm_tile_grid(p), s);
+}
+
+template <int EPI>
+int gemm_digits_t(const GemmP &p, hipStream_t s) {
+    // the smaller tiles write SwiGLU as f32 rows only
+    const CutPick d = pick_cut(kDigitTiles, EPI != GE_SWIGLU || p.of ? 6 : 1, p.M, p.N, p.nk, sizeof(double), 16);
+    if (!d.cols) return gemm_digits_tile<EPI>(p, d.first, s);
+    SCRY_TRY(gemm_digits_tile<EPI>(gemm_cols(p, 0, d.cols, 1), d.first, s));
+    return gemm_digits_tile<EPI>(gemm_cols(p, d.cols, p.N - d.cols, 1), d.rest, s);
 }
 
 template <int EPI, bool WBF, bool B32, class C>
@@ -1860,13 +1917,9 @@ int ring_small(GemmP p, int splits, hipStream_t s) {
     return SCRY_OK;
 }
 
-// WBF or B32: the tile by pick_tile; int8 per-tensor weights through bf16
-// planes (k beyond the digit kernel's): the large tile
-template <int EPI, bool WBF, bool B32 = false>
-int gemm_ring_t(const GemmP &p, hipStream_t s) {
+template <int EPI, bool WBF, bool B32>
+int gemm_ring_tile(const GemmP &p, const TilePick &d, hipStream_t s) {
     if constexpr (WBF || B32) {
-        // SwiGLU planes come from the whole sums: no k splits
-        const TilePick d = pick_tile(B32 ? kB32Tiles : kRingTiles, p.M, p.N, p.nk, sizeof(float), 5, EPI == GE_SWIGLU ? 1 : 8);
         switch (d.tile) {
             case 1: return ring_small<EPI, WBF, B32, RTile<WBF, B32, 128, 128, 2, 4, 3>>(p, d.splits, s);
             case 2: return ring_small<EPI, WBF, B32, RTile<WBF, B32, 64, 128, 2, 2, 3>>(p, d.splits, s);
@@ -1875,6 +1928,18 @@ int gemm_ring_t(const GemmP &p, hipStream_t s) {
         }
     }
     return ring_launch<EPI, WBF, B32, RBig<WBF, B32>>(p, gemm_tile_grid(p), s);
+}
+
+// WBF or B32: the tile by pick_cut; int8 per-tensor weights through bf16
+// planes (k beyond the digit kernel's): the large tile
+template <int EPI, bool WBF, bool B32 = false>
+int gemm_ring_t(const GemmP &p, hipStream_t s) {
+    if (!WBF && !B32) return gemm_ring_tile<EPI, WBF, B32>(p, {0, 1, 0.0}, s);
+    // SwiGLU planes come from the whole sums: no k splits
+    const CutPick d = pick_cut(B32 ? kB32Tiles : kRingTiles, 5, p.M, p.N, p.nk, sizeof(float), EPI == GE_SWIGLU ? 1 : 8);
+    if (!d.cols) return gemm_ring_tile<EPI, WBF, B32>(p, d.first, s);
+    SCRY_TRY((gemm_ring_tile<EPI, WBF, B32>(gemm_cols(p, 0, d.cols, WBF ? 2 : 1), d.first, s)));
+    return gemm_ring_tile<EPI, WBF, B32>(gemm_cols(p, d.cols, p.N - d.cols, WBF ? 2 : 1), d.rest, s);
 }
 
 }  // namespace

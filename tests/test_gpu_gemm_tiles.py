@@ -12,7 +12,8 @@ F = np.float32
 @pytest.mark.parametrize("m,k,n", [
     (17, 64, 5), (33, 100, 131), (32, 2048, 128), (37, 4096, 260), (64, 768, 768), (65, 3072, 770),
     (130, 4096, 1030), (200, 768, 2304), (129, 8192, 4096), (300, 1024, 4097), (512, 2048, 2050),
-    (129, 256, 28416), (600, 128, 28000), (255, 192, 21889), (1100, 64, 13000)])
+    (129, 256, 28416), (600, 128, 28000), (255, 192, 21889), (1100, 64, 13000),
+    (384, 1100, 22018), (600, 1024, 14339), (1500, 1024, 6145), (511, 2048, 22013)])
 def test_exact_sums(hip, m, k, n):
     print(f"[case] {m} x {k} x {n}", flush=True)
     B = hip.HipBackend
@@ -58,9 +59,32 @@ def test_prefill_with_split_k_matches_decode(hip, seq):
     m.free()
 
 
+@pytest.mark.parametrize("mode", ["per_tensor", "block32", "bf16"])
+@pytest.mark.parametrize("seq,ffn", [(600, 7172), (384, 11004)])
+def test_prefill_in_two_launches_matches_shorter(hip, mode, seq, ffn):
+    """SwiGLU columns cut into two launches (full rounds of the chip, the rest):
+    one prompt, against the same prompt in pieces of 100 rows, which need no
+    cut.  Tolerances as the tests against the decode path."""
+    print(f"[case] {mode} seq={seq} ffn={ffn}", flush=True)
+    import esolearn_amd.llama as EL
+    q = {"per_tensor": EL.QUANT_PER_TENSOR, "block32": EL.QUANT_BLOCK32, "bf16": EL.QUANT_BF16}[mode]
+    cfg = hip.LlamaConfig(vocab_size=96, hidden_size=2048, intermediate_size=ffn, n_layers=2, n_heads=16,
+                          n_kv_heads=4, max_seq_len=640, rope_theta=10000.0, tie_word_embeddings=False)
+    m = hip.LlamaModel.new_random(cfg, 3, quant_mode=q, init_on_device=True)
+    toks = np.random.default_rng(seq).integers(0, 96, seq)
+    ca, cb = m.new_llama_kv_cache(seq + 1), m.new_llama_kv_cache(seq + 1)
+    m.prefill([ca], toks[None, :])
+    for at in range(0, seq, 100):
+        m.prefill([cb], toks[None, at:at + 100])
+    a, _ = m.forward_with_llama_cache(5, seq, ca)  # reads every row of both layers' caches
+    b, _ = m.forward_with_llama_cache(5, seq, cb)
+    assert np.abs(a - b).max() <= (1e-2 if mode == "bf16" else 1e-3) * np.abs(b).max()
+    m.free()
+
+
 @pytest.mark.parametrize("m,k,n", [
     (17, 64, 5), (37, 100, 131), (32, 4096, 260), (64, 768, 768), (130, 4096, 1030), (200, 3072, 770),
-    (129, 1280, 5120), (300, 1024, 4097), (512, 8192, 1024)])
+    (129, 1280, 5120), (300, 1024, 4097), (512, 8192, 1024), (600, 2048, 14339)])
 def test_bf16_exact_sums(hip, m, k, n):
     """The bf16 GEMM's tiles and splits: integers exact in bf16, sums exact in f32."""
     print(f"[case] bf16 {m} x {k} x {n}", flush=True)
@@ -98,7 +122,7 @@ def test_bf16_prefill_small_tiles_match_decode(hip, seq):
 
 @pytest.mark.parametrize("m,k,n", [
     (17, 64, 5), (33, 100, 131), (40, 4096, 260), (64, 768, 768), (130, 3000, 1030), (129, 4096, 4096),
-    (300, 1024, 4097), (512, 11008, 516)])
+    (300, 1024, 4097), (512, 11008, 516), (600, 1024, 14339)])
 def test_block32_exact_sums(hip, m, k, n):
     """Block-32 scales that are powers of two: every product and sum is exact in f32."""
     print(f"[case] block32 {m} x {k} x {n}", flush=True)

@@ -49,12 +49,14 @@ constexpr int MM_T = 256, MM_BK = 32, MM_S = 36;
 // The f64 MFMA leaves hardly any issue slots to other vector instructions
 // (counters: with 6 of them per MFMA the matrix cores were 58% busy), so the
 // step loop has no branches and no clamps: a step's loads are buffer loads
-// from a uniform base that the step moves, per-thread offsets are computed
-// once, and the range check zeroes k positions past the range (rows of
-// [k][row]: the resource ends there; [row][k]: the offset is replaced by one
-// past every resource).  LD_QUAD reads 16 bytes along k (k % 4 == 0), LD_WORD
-// single values; LD_WIDE is for matrices whose offsets inside a tile do not
-// fit 31 bits.
+// from uniform bases that the step moves, per-thread offsets are computed
+// once, and the range check zeroes k positions past the range.  [row][k]: the
+// offset is replaced by one past every resource.  [k][row]: k position 4 q + u
+// goes through a resource of u's own, which starts at k row u and ends with the
+// range (scalar instructions only: as fast as one resource and a scalar offset
+// of u rows, which the compiler leaves out of what the range check promises).
+// LD_QUAD reads 16 bytes along k (k % 4 == 0), LD_WORD single values; LD_WIDE
+// is for matrices whose offsets inside a tile do not fit 31 bits.
 enum { LD_WIDE = 0, LD_WORD = 1, LD_QUAD = 2 };
 
 template <int R, bool KC, int LD>
@@ -101,24 +103,35 @@ struct Stage {
             }
             return;
         }
-        const size_t first = KC ? (size_t)r0 * k + k0 : (size_t)k0 * rows + r0;
         // values left up to the end, capped at the resource limit (scalar 32-bit compares)
-        const long long d = (long long)((size_t)rows * (KC ? k : kend) - first);
-        const int hi = (int)(d >> 29), nb = hi < 0 ? 0 : hi > 0 ? 0x7ffffffc : (int)d * 4;
-        const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p) + first, (short)0, nb, 0x00020000);
-        constexpr unsigned past = 0x80000000u;
+        auto rsrc = [&](size_t first) {
+            const long long d = (long long)((size_t)rows * (KC ? k : kend) - first);
+            const int hi = (int)(d >> 29), nb = hi < 0 ? 0 : hi > 0 ? 0x7ffffffc : (int)d * 4;
+            return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p) + first, (short)0, nb, 0x00020000);
+        };
+        if (KC) {
+            constexpr unsigned past = 0x80000000u;
+            const auto rs = rsrc((size_t)r0 * k + k0);
 #pragma unroll
-        for (int j = 0; j < N; j++) {
-            int row, q;
-            slot(j, row, q);
-            if (KC && LD == LD_QUAD) {
-                v[j] = dev::bload16f(rs, left > 4 * q ? off[j] : past);
-            } else {
+            for (int j = 0; j < N; j++) {
+                int row, q;
+                slot(j, row, q);
+                if (LD == LD_QUAD) {
+                    v[j] = dev::bload16f(rs, left > 4 * q ? off[j] : past);
+                } else {
 #pragma unroll
-                for (int u = 0; u < 4; u++)
-                    (&v[j].x)[u] = __builtin_bit_cast(
-                        float, KC ? __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(left > 4 * q + u ? off[j] + 4 * u : past), 0, 0)
-                                  : __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off[j], 4 * u * rows, 0));
+                    for (int u = 0; u < 4; u++)
+                        (&v[j].x)[u] = __builtin_bit_cast(
+                            float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(left > 4 * q + u ? off[j] + 4 * u : past), 0, 0));
+                }
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const auto rs = rsrc((size_t)(k0 + u) * rows + r0);
+#pragma unroll
+                for (int j = 0; j < N; j++)
+                    (&v[j].x)[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off[j], 0, 0));
             }
         }
     }

@@ -13,7 +13,7 @@ F = np.float32
 SHAPES = [  # batch, m, k, n
     (1, 1, 1, 1), (2, 1, 129, 77), (32, 1, 101, 128), (1, 2, 1001, 12), (3, 3, 33, 70), (1, 4, 4100, 260),
     (1, 1, 2048, 4100), (1, 5, 3, 7), (2, 33, 31, 65), (3, 17, 100, 129), (1, 37, 128, 37), (1, 200, 768, 50),
-    (1, 65, 2052, 68), (1, 70, 4097, 66), (12, 64, 64, 64), (1, 1030, 70, 1029),
+    (1, 65, 2052, 68), (1, 70, 4097, 66), (2, 70, 33, 66), (12, 64, 64, 64), (1, 1030, 70, 1029),
 ]
 
 
@@ -61,3 +61,33 @@ def test_matmul_nonfinite_stays_in_its_rows_and_columns(hip, m, ta, tb):
     with np.errstate(invalid="ignore"):
         ref = (a.astype(np.float64) @ b.astype(np.float64)).astype(F)
     assert np.array_equal(np.isnan(c), np.isnan(ref)) and np.array_equal(np.isinf(c), np.isinf(ref))
+
+
+def _block_bytes(n):
+    """The pool's size class of an n-byte storage: (8 + i) << (e + 5) bytes."""
+    return next(c for e in range(40) for c in ((8 + i) << (e + 5) for i in range(8)) if c >= n)
+
+
+@pytest.mark.parametrize("k", [33, 34, 35, 65, 4097])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_matmul_reads_nothing_past_a_matrix(hip, k, ta, tb):
+    """What lies behind the k tail of an operand - the next batch entry, and
+    after the last entry the rest of its storage block - is NaN: no product may
+    take it up (a tail position times a stale NaN would show)."""
+    print(f"[case] k={k} ta={ta} tb={tb}", flush=True)
+    B = hip.HipBackend
+    bt, m, n = 3, 70, 66
+    rng = np.random.default_rng(k + 2 * ta + tb)
+    a = rng.normal(size=(bt, m, k)).astype(F)
+    b = rng.normal(size=(bt, k, n)).astype(F)
+    a[1] = np.nan  # entry 0 borders on it, entry 2 on the rest of the block
+    b[1] = np.nan
+
+    def storage(x):  # in a block that was all NaN before
+        B.from_vec(np.full(_block_bytes(x.nbytes) // 4, np.nan, F)).free()
+        return B.from_vec(np.ascontiguousarray(x))
+
+    A, W = storage(a.swapaxes(1, 2) if ta else a), storage(b.swapaxes(1, 2) if tb else b)
+    c = B.matmul_strided_batched(A, W, bt, m, k, n, bool(ta), bool(tb)).to_vec().reshape(bt, m, n)
+    assert np.isnan(c[1]).all()
+    _check(c[::2], a[::2], b[::2])

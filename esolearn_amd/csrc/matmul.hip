@@ -22,8 +22,9 @@ struct MMArgs {
     const float *a, *b, *bias;  // bias [n] or null (added in f32 to the rounded sum)
     float *c;
     double *part;  // splits > 1: f64 partial sums [split][batch][m][n]
-    int batch, m, k, n, splits, kchunk;
-    int tm, tn;      // tiles
+    int batch, m, k, n, splits;
+    unsigned kchunk;
+    int tm, tn;  // tiles
 };
 
 // ---------------------------------------------------------------- matrix cores
@@ -59,8 +60,20 @@ constexpr int MM_T = 256, MM_BK = 32, MM_S = 36;
 // is for matrices whose offsets inside a tile do not fit 31 bits.
 enum { LD_WIDE = 0, LD_WORD = 1, LD_QUAD = 2 };
 
+// k positions, and rows and columns at a tile's end: above the LD_WIDE limit
+// they may pass 2^31 - 1
+template <int LD>
+struct Index {
+    typedef int T;
+};
+template <>
+struct Index<LD_WIDE> {
+    typedef unsigned T;
+};
+
 template <int R, bool KC, int LD>
 struct Stage {
+    typedef typename Index<LD>::T K;
     static constexpr int N = R * MM_BK / 4 / MM_T;  // float4 per thread
     float4 v[N];
     unsigned off[N];   // bytes from the tile's first row (KC) or column at the step's k
@@ -86,32 +99,33 @@ struct Stage {
     // the values of step [k0, k0 + 32) of a range that ends at kend; none of
     // them is used here, or the wave would wait for the loads before the
     // MFMAs that are to hide them
-    __device__ __forceinline__ void load(const float *p, int rows, int k, int r0, int k0, int kend) {
-        const int left = kend - k0;
+    __device__ __forceinline__ void load(const float *p, int rows, int k, int r0, K k0, K kend) {
+        const int left = (int)(kend - k0);
         if (LD == LD_WIDE) {
 #pragma unroll
             for (int j = 0; j < N; j++) {
                 int row, q;
                 slot(j, row, q);
-                const int r = min(r0 + row, rows - 1);
+                const unsigned r = min((unsigned)(r0 + row), (unsigned)(rows - 1));
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    const int c = min(k0 + 4 * q + u, k - 1);
+                    const K c = min(k0 + 4 * q + u, (K)(k - 1));
                     const float y = KC ? p[(size_t)r * k + c] : p[(size_t)c * rows + r];
                     (&v[j].x)[u] = left > 4 * q + u ? y : 0.f;
                 }
             }
             return;
         }
-        // values left up to the end, capped at the resource limit (scalar 32-bit compares)
-        auto rsrc = [&](size_t first) {
-            const long long d = (long long)((size_t)rows * (KC ? k : kend) - first);
-            const int hi = (int)(d >> 29), nb = hi < 0 ? 0 : hi > 0 ? 0x7ffffffc : (int)d * 4;
+        auto rsrc = [&](size_t first, int nb) {
             return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p) + first, (short)0, nb, 0x00020000);
         };
         if (KC) {
             constexpr unsigned past = 0x80000000u;
-            const auto rs = rsrc((size_t)r0 * k + k0);
+            // values left up to the end, capped at the resource limit (scalar 32-bit compares)
+            const size_t first = (size_t)r0 * k + k0;
+            const long long d = (long long)((size_t)rows * k - first);
+            const int hi = (int)(d >> 29);
+            const auto rs = rsrc(first, hi < 0 ? 0 : hi > 0 ? 0x7ffffffc : (int)d * 4);
 #pragma unroll
             for (int j = 0; j < N; j++) {
                 int row, q;
@@ -126,9 +140,12 @@ struct Stage {
                 }
             }
         } else {
+            // k rows of this step inside the range, from row r0 of the first on
+            const int here = min(left, MM_BK) * rows - r0;  // below 2^26 (2^21 rows or columns at most)
+            const size_t first = (size_t)k0 * rows + r0;
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const auto rs = rsrc((size_t)(k0 + u) * rows + r0);
+                const auto rs = rsrc(first + (size_t)u * rows, 4 * max(here - u * rows, 0));
 #pragma unroll
                 for (int j = 0; j < N; j++)
                     (&v[j].x)[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off[j], 0, 0));
@@ -164,7 +181,8 @@ __global__ __launch_bounds__(MM_T, 2) void k_mm_f64(MMArgs p) {
     const int sp = (int)(w / ((unsigned)p.tm * p.tn) % p.splits), bt = (int)(w / ((unsigned)p.tm * p.tn * p.splits));
     const float *A = p.a + (size_t)bt * p.m * p.k, *B = p.b + (size_t)bt * p.k * p.n;
     const int i0 = it * BM, j0 = jt * BN;
-    const int kb = sp * p.kchunk, ke = min(p.k, kb + p.kchunk);
+    typedef typename Index<LD>::T K;
+    const K kb = (K)sp * (K)p.kchunk, ke = min((K)p.k, kb + (K)p.kchunk);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = (wave & 1) * WM, wn = (wave >> 1) * WN;
     const int fo = (lane & 15) * MM_S + 4 * (lane >> 4);
@@ -183,7 +201,7 @@ __global__ __launch_bounds__(MM_T, 2) void k_mm_f64(MMArgs p) {
     lb.store(sb[0]);
     __syncthreads();
     int cur = 0;
-    for (int k0 = kb; k0 < ke; k0 += MM_BK) {
+    for (K k0 = kb; k0 < ke; k0 += MM_BK) {
         la.load(A, p.m, p.k, i0, k0 + MM_BK, ke);
         lb.load(B, p.n, p.k, j0, k0 + MM_BK, ke);
 #pragma unroll
@@ -221,11 +239,11 @@ __global__ __launch_bounds__(MM_T, 2) void k_mm_f64(MMArgs p) {
     for (int x = 0; x < NM; x++)
 #pragma unroll
         for (int y = 0; y < NN; y++) {
-            const int j = j0 + wn + 16 * y + ci;
+            const K j = (K)j0 + wn + 16 * y + ci;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int i = i0 + wm + 16 * x + 4 * r + cg;
-                if (i >= p.m || j >= p.n) continue;
+                const K i = (K)i0 + wm + 16 * x + 4 * r + cg;
+                if (i >= (K)p.m || j >= (K)p.n) continue;
                 const size_t o = (size_t)i * p.n + j;
                 if (p.splits > 1) {
                     p.part[((size_t)sp * p.batch + bt) * mn + o] = acc[x][y][r];
@@ -273,7 +291,7 @@ __global__ __launch_bounds__(256) void k_mv_rows(const float *__restrict__ a, co
         for (int i = 0; i < MT; i++) acc[r][i] = 0.0;
     constexpr int W = VEC ? 4 : 1;
 #pragma unroll 2
-    for (int p = l * W; p < k; p += G * W) {
+    for (unsigned p = l * W; p < (unsigned)k; p += G * W) {  // unsigned: k may be 2^31 - 1
         float bv[MV_R][W], av[MT][W];
 #pragma unroll
         for (int r = 0; r < MV_R; r++) {
@@ -322,7 +340,7 @@ __global__ __launch_bounds__(256) void k_mv_rows(const float *__restrict__ a, co
 template <int MT, int W>
 __global__ __launch_bounds__(256) void k_mv_cols(const float *__restrict__ a, const float *__restrict__ b,
                                                  const float *__restrict__ bias, int batch, int m, int k, int n,
-                                                 int ta, int cg, int splits, int kchunk, float *__restrict__ c,
+                                                 int ta, int cg, int splits, unsigned kchunk, float *__restrict__ c,
                                                  double *__restrict__ part) {
     __shared__ double red[MT * W * 256];
     const int bt = blockIdx.z, sp = blockIdx.y, kg = 256 / cg;
@@ -330,18 +348,18 @@ __global__ __launch_bounds__(256) void k_mv_cols(const float *__restrict__ a, co
     const int j0 = (blockIdx.x * cg + tc) * W;
     const float *A = a + (size_t)bt * m * k;
     const float *B = b + (size_t)bt * k * n + min(j0, n - W);
-    const int kb = sp * kchunk, ke = min(k, kb + kchunk);
+    const unsigned kb = sp * kchunk, ke = min((unsigned)k, kb + kchunk);
     double acc[MT][W];
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
         for (int u = 0; u < W; u++) acc[i][u] = 0.0;
     constexpr int U = 8;  // rows in flight
-    for (int p0 = kb + tk; p0 < ke; p0 += U * kg) {
+    for (unsigned p0 = kb + tk; p0 < ke; p0 += U * kg) {
         float bv[U][W], av[U][MT];
 #pragma unroll
         for (int q = 0; q < U; q++) {
-            const int p = min(p0 + q * kg, ke - 1);
+            const unsigned p = min(p0 + q * kg, ke - 1);
             if (W == 4)
                 *reinterpret_cast<float4 *>(bv[q]) = *reinterpret_cast<const float4 *>(B + (size_t)p * n);
             else
@@ -439,8 +457,8 @@ int mv_cols(const float *a, const float *b, const float *bias, int batch, int m,
     // about 1024 workgroups (4 per CU), each k group at least 16 rows
     int splits = (1024 + cb * batch - 1) / (cb * batch);
     splits = std::max(1, std::min({splits, k / (16 * kg), 64}));
-    const int kchunk = (k + splits - 1) / splits;
-    splits = (k + kchunk - 1) / kchunk;
+    const unsigned kchunk = ((unsigned)k + splits - 1) / splits;
+    splits = (int)(((unsigned)k + kchunk - 1) / kchunk);
     void *ws = nullptr;
     if (splits > 1) SCRY_TRY(ctx_workspace(sizeof(double) * (size_t)splits * batch * m * n, &ws));
     const dim3 g(cb, splits, batch);
@@ -479,20 +497,21 @@ int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, i
     p.m = m;
     p.k = k;
     p.n = n;
-    auto tiles = [&](int t) { return (size_t)batch * ((m + t - 1) / t) * ((n + t - 1) / t); };
-    const bool wide = std::max({m, n, k}) > (1 << 21);  // 31-bit offsets: 128 rows of k, or 32 k rows of m or n values
+    auto tile_count = [](int x, int t) { return (int)(((unsigned)x + t - 1) / t); };
+    auto tiles = [&](int t) { return (size_t)batch * tile_count(m, t) * tile_count(n, t); };
+    const bool wide = std::max({m, n, k}) > (1 << 21);  // 31-bit offsets: 64 rows of k, or 32 k rows of m or n values
     // 64 x 64 tiles where they fill the CUs or a long k can be split over
     // them, else 32 x 32 (12 x 200 x 200 x 64: 6 against 14 us; 64 x 4096 x
     // 4096, split: 62 against 49 us).  128 x 128 was slower everywhere
     // (1500 x 1280 x 5120: 513 against 368 us, one wave per SIMD).
-    const int steps = (k + MM_BK - 1) / MM_BK;
+    const int steps = tile_count(k, MM_BK);
     const int t = tiles(64) >= 256 || (steps >= 64 && m > 32 && n > 32) ? 64 : 32;
-    p.tm = (m + t - 1) / t;
-    p.tn = (n + t - 1) / t;
+    p.tm = tile_count(m, t);
+    p.tn = tile_count(n, t);
     const size_t nt = tiles(t);
     p.splits = nt >= 512 ? 1 : (int)std::max<size_t>(1, std::min<size_t>({(512 + nt - 1) / nt, (size_t)steps / 8, 16}));
     const int cs = (steps + p.splits - 1) / p.splits;
-    p.kchunk = cs * MM_BK;
+    p.kchunk = (unsigned)cs * MM_BK;
     p.splits = (steps + cs - 1) / cs;
     if (p.splits > 1) {
         void *ws = nullptr;

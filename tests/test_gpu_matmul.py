@@ -91,3 +91,43 @@ def test_matmul_reads_nothing_past_a_matrix(hip, k, ta, tb):
     c = B.matmul_strided_batched(A, W, bt, m, k, n, bool(ta), bool(tb)).to_vec().reshape(bt, m, n)
     assert np.isnan(c[1]).all()
     _check(c[::2], a[::2], b[::2])
+
+
+TOP = 2 ** 31 - 1  # the largest dimension an entry point takes
+
+
+@pytest.mark.parametrize("m,k,n,tb", [(1, TOP, 1, 1), (1, TOP - 31, 1, 0), (5, TOP, 1, 1), (TOP, 1, 1, 0), (1, 1, TOP, 0)])
+def test_matmul_largest_dimension(hip, m, k, n, tb):
+    """A dimension whose last tile or stride ends past 2^31 - 1.  Products of
+    ones: the f64 sums are exact, so a position left out or taken twice shows."""
+    print(f"[case] {m} x {k} x {n} tb={tb}", flush=True)
+    B = hip.HipBackend
+    c = B.matmul(B.ones(m * k), B.ones(k * n), m, k, n, False, bool(tb))
+    if m * n < 100:
+        assert (c.to_vec() == F(k)).all()
+    else:
+        assert c.n == m * n and B.sum(c) == F(m * n)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,k,n", [(5, 33, 2 ** 21 + 41), (2 ** 21 + 41, 33, 5), (6, 2 ** 21 + 41, 7)])
+def test_matmul_wide(hip, m, k, n, ta, tb):
+    """A dimension above 2^21: loads with 64-bit addresses."""
+    print(f"[case] {m} x {k} x {n} ta={ta} tb={tb}", flush=True)
+    B = hip.HipBackend
+    rng = np.random.default_rng(m + k + n)
+    a = rng.normal(size=(1, m, k)).astype(F)
+    b = rng.normal(size=(1, k, n)).astype(F)
+    A = B.from_vec(np.ascontiguousarray(a.swapaxes(1, 2) if ta else a))
+    W = B.from_vec(np.ascontiguousarray(b.swapaxes(1, 2) if tb else b))
+    _check(B.matmul(A, W, m, k, n, bool(ta), bool(tb)).to_vec().reshape(1, m, n), a, b)
+
+
+def test_matmul_more_tiles_than_workgroups(hip):
+    """2^22 + 9 batch entries: a workgroup takes several tiles."""
+    B = hip.HipBackend
+    bt, m, k, n = 2 ** 22 + 9, 2, 3, 2
+    rng = np.random.default_rng(5)
+    a = rng.normal(size=(bt, m, k)).astype(F)
+    b = rng.normal(size=(bt, k, n)).astype(F)
+    _check(B.matmul_strided_batched(B.from_vec(a), B.from_vec(b), bt, m, k, n).to_vec().reshape(bt, m, n), a, b)

@@ -73,6 +73,15 @@ int ctx_workspace(size_t bytes, void **p) {
     return SCRY_OK;
 }
 
+int split_workspace(size_t bytes, int *splits, void **p) {
+    *p = nullptr;
+    if (*splits <= 1) return SCRY_OK;
+    const int rc = ctx_workspace(bytes * *splits, p);
+    if (rc != SCRY_ERR_OOM) return rc;
+    *splits = 1;
+    return SCRY_OK;
+}
+
 void dev_free(void *p) {
     if (p) (void)hipFree(p);
 }

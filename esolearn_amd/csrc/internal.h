@@ -28,6 +28,9 @@ Ctx &ctx();
 // The context's workspace, at least `bytes` large.  Work already queued on
 // the stream may still use the old one, so growing it synchronises first.
 int ctx_workspace(size_t bytes, void **p);
+// The workspace for the partial sums of *splits k splits, `bytes` each; where
+// the device has no memory left for it *splits becomes 1: the work runs whole.
+int split_workspace(size_t bytes, int *splits, void **p);
 std::recursive_mutex &api_mutex();
 
 int set_error(int code, const char *fmt, ...);

@@ -405,6 +405,9 @@ __global__ __launch_bounds__(256) void k_mv_cols(const float *__restrict__ a, co
 
 #define LAUNCH_CHECK() SCRY_HIP(hipGetLastError()); return SCRY_OK
 
+// parts of p (1 or more) that cover x > 0
+unsigned parts(unsigned x, unsigned p) { return (x + p - 1) / p; }
+
 int reduce_parts(const double *part, int splits, size_t total, int n, const float *bias, float *c, hipStream_t s) {
     const size_t g = (total + 255) / 256;
     hipLaunchKernelGGL(k_mm_reduce, dim3((unsigned)(g > 65536 ? 65536 : g)), dim3(256), 0, s, part, splits, total, n,
@@ -457,10 +460,10 @@ int mv_cols(const float *a, const float *b, const float *bias, int batch, int m,
     // about 1024 workgroups (4 per CU), each k group at least 16 rows
     int splits = (1024 + cb * batch - 1) / (cb * batch);
     splits = std::max(1, std::min({splits, k / (16 * kg), 64}));
-    const unsigned kchunk = ((unsigned)k + splits - 1) / splits;
-    splits = (int)(((unsigned)k + kchunk - 1) / kchunk);
+    splits = (int)parts(k, parts(k, splits));  // none empty
     void *ws = nullptr;
-    if (splits > 1) SCRY_TRY(ctx_workspace(sizeof(double) * (size_t)splits * batch * m * n, &ws));
+    SCRY_TRY(split_workspace(sizeof(double) * (size_t)batch * m * n, &splits, &ws));
+    const unsigned kchunk = parts(k, splits);
     const dim3 g(cb, splits, batch);
     if (W == 4)
         hipLaunchKernelGGL((k_mv_cols<MT, 4>), g, dim3(256), 0, s, a, b, bias, batch, m, k, n, ta, cg, splits, kchunk,
@@ -497,27 +500,23 @@ int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, i
     p.m = m;
     p.k = k;
     p.n = n;
-    auto tile_count = [](int x, int t) { return (int)(((unsigned)x + t - 1) / t); };
-    auto tiles = [&](int t) { return (size_t)batch * tile_count(m, t) * tile_count(n, t); };
+    auto tiles = [&](int t) { return (size_t)batch * parts(m, t) * parts(n, t); };
     const bool wide = std::max({m, n, k}) > (1 << 21);  // 31-bit offsets: 64 rows of k, or 32 k rows of m or n values
     // 64 x 64 tiles where they fill the CUs or a long k can be split over
     // them, else 32 x 32 (12 x 200 x 200 x 64: 6 against 14 us; 64 x 4096 x
     // 4096, split: 62 against 49 us).  128 x 128 was slower everywhere
     // (1500 x 1280 x 5120: 513 against 368 us, one wave per SIMD).
-    const int steps = tile_count(k, MM_BK);
+    const int steps = (int)parts(k, MM_BK);
     const int t = tiles(64) >= 256 || (steps >= 64 && m > 32 && n > 32) ? 64 : 32;
-    p.tm = tile_count(m, t);
-    p.tn = tile_count(n, t);
+    p.tm = (int)parts(m, t);
+    p.tn = (int)parts(n, t);
     const size_t nt = tiles(t);
     p.splits = nt >= 512 ? 1 : (int)std::max<size_t>(1, std::min<size_t>({(512 + nt - 1) / nt, (size_t)steps / 8, 16}));
-    const int cs = (steps + p.splits - 1) / p.splits;
-    p.kchunk = (unsigned)cs * MM_BK;
-    p.splits = (steps + cs - 1) / cs;
-    if (p.splits > 1) {
-        void *ws = nullptr;
-        SCRY_TRY(ctx_workspace(sizeof(double) * (size_t)p.splits * batch * m * n, &ws));
-        p.part = (double *)ws;
-    }
+    p.splits = (int)parts(steps, parts(steps, p.splits));  // none empty
+    void *ws = nullptr;
+    SCRY_TRY(split_workspace(sizeof(double) * (size_t)batch * m * n, &p.splits, &ws));
+    p.part = (double *)ws;
+    p.kchunk = parts(steps, p.splits) * MM_BK;
     if (wide)
         t == 32 ? mm_launch<32, LD_WIDE>(p, ta, tb, s) : mm_launch<64, LD_WIDE>(p, ta, tb, s);
     else if (k % 4 == 0)

@@ -1754,17 +1754,22 @@ int digits_launch(const GemmP &p, int grid, hipStream_t s) {
     PF_LAUNCH_CHECK();
 }
 
+// p's k splits, none empty, and the workspace of their partial sums (el bytes each)
+int set_splits(GemmP &p, int splits, size_t el, void **ws) {
+    p.kchunk = (p.nk + splits - 1) / splits;
+    p.splits = (p.nk + p.kchunk - 1) / p.kchunk;
+    SCRY_TRY(split_workspace(el * p.M * p.N, &p.splits, ws));
+    if (p.splits == 1) p.kchunk = p.nk;
+    return SCRY_OK;
+}
+
 template <int EPI, class TL>
 int digits_small(GemmP p, int splits, hipStream_t s) {
     p.n_mb = (p.M + TL::BM - 1) / TL::BM;
     p.n_nb = (p.N + TL::BN - 1) / TL::BN;
-    p.kchunk = (p.nk + splits - 1) / splits;
-    p.splits = (p.nk + p.kchunk - 1) / p.kchunk;
-    if (p.splits > 1) {
-        void *ws = nullptr;
-        SCRY_TRY(ctx_workspace(sizeof(double) * (size_t)p.splits * p.M * p.N, &ws));
-        p.part = (double *)ws;
-    }
+    void *ws = nullptr;
+    SCRY_TRY(set_splits(p, splits, sizeof(double), &ws));
+    p.part = (double *)ws;
     SCRY_TRY((digits_launch<EPI, TL>(p, (p.n_mb * p.n_nb * p.splits + 7) / 8 * 8, s)));
     if (p.splits > 1) {
         const size_t g = ((size_t)p.M * ((p.N + 3) / 4) + 255) / 256;
@@ -1901,13 +1906,9 @@ template <int EPI, bool WBF, bool B32, class C>
 int ring_small(GemmP p, int splits, hipStream_t s) {
     p.n_mb = (p.M + C::BM - 1) / C::BM;
     p.n_nb = (p.N + C::BN - 1) / C::BN;
-    p.kchunk = (p.nk + splits - 1) / splits;
-    p.splits = (p.nk + p.kchunk - 1) / p.kchunk;
-    if (p.splits > 1) {
-        void *ws = nullptr;
-        SCRY_TRY(ctx_workspace(sizeof(float) * (size_t)p.splits * p.M * p.N, &ws));
-        p.partf = (float *)ws;
-    }
+    void *ws = nullptr;
+    SCRY_TRY(set_splits(p, splits, sizeof(float), &ws));
+    p.partf = (float *)ws;
     SCRY_TRY((ring_launch<EPI, WBF, B32, C>(p, (p.n_mb * p.n_nb * p.splits + 7) / 8 * 8, s)));
     if (p.splits > 1) {
         const size_t g = ((size_t)p.M * p.N + 255) / 256;

@@ -1,4 +1,5 @@
 import os
+import subprocess
 import sys
 
 import pytest
@@ -32,3 +33,36 @@ def hip():
     info = E.HipBackend.device_info()
     print(f"[gpu] {info}", flush=True)
     return E
+
+
+FAKE_PRELUDE = """
+import ctypes as C, sys
+import numpy as np
+import esolearn_amd as E
+F = C.CDLL(sys.argv[1])
+F.fake_used.restype = C.c_size_t
+F.fake_limit.argtypes = [C.c_size_t]
+F.fake_launches.restype = C.c_char_p
+def launches():
+    return F.fake_launches().decode().splitlines()
+E.init(0)
+B = E.HipBackend
+"""
+
+
+@pytest.fixture(scope="session")
+def fake_hip(tmp_path_factory):
+    """Runs Python code in a fresh process on tests/fake_hip.cpp (a runtime
+    without a device: host logic only, kernels are recorded and not run)."""
+    lib = str(tmp_path_factory.mktemp("fake_hip") / "fake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-fPIC", "-shared",
+                    os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", lib], check=True)
+
+    def run(code):
+        pre = " ".join(x for x in (lib, os.environ.get("LD_PRELOAD")) if x)
+        r = subprocess.run([sys.executable, "-c", FAKE_PRELUDE + code, lib], capture_output=True, text=True, timeout=300,
+                           cwd=ROOT, env={**os.environ, "LD_PRELOAD": pre})
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+
+    return run

@@ -122,6 +122,15 @@ void del_buf(scry_buf b) {
     delete b;
 }
 
+// a failed op leaves no output behind
+int keep_out(int rc, scry_buf *out) {
+    if (rc) {
+        del_buf(*out);
+        *out = nullptr;
+    }
+    return rc;
+}
+
 // the f32 data changed in place: drop the bf16 copies made from it
 void bf16_stale(scry_buf b) {
     if (!b->d) return;
@@ -223,11 +232,7 @@ int matmul_bf16(scry_buf a, scry_buf b, int m, int k, int n, int ta, int tb, scr
     pool_free(tmp);
     pool_free(tb_f);
     pool_free(plane);
-    if (rc) {
-        del_buf(*out);
-        *out = nullptr;
-    }
-    return rc;
+    return keep_out(rc, out);
 }
 
 // Ensure the GEMV layout of an I8Storage for logical [k, n].
@@ -706,7 +711,7 @@ int scry_hip_matmul(scry_buf a, scry_buf b, int m, int k, int n, int trans_a, in
     CHECK_BUF(b, "matmul");
     SCRY_TRY(check_mkn(a->n, b->n, m, k, n));
     SCRY_TRY(new_buf((size_t)m * n, out));
-    return launch_matmul_f32(a->d, b->d, 1, m, k, n, trans_a, trans_b, nullptr, (*out)->d, ctx().stream);
+    return keep_out(launch_matmul_f32(a->d, b->d, 1, m, k, n, trans_a, trans_b, nullptr, (*out)->d, ctx().stream), out);
 }
 
 // MathBackend::matmul_bias (mod.rs:62-86; the CUDA backend keeps the default):
@@ -737,11 +742,7 @@ int scry_hip_matmul_bias(scry_buf a, scry_buf b, scry_buf bias, int m, int k, in
         if (!rc) rc = launch_matmul_f32(a->d, b->d, 1, m, k, n, trans_a, trans_b, bv, (*out)->d, ctx().stream);
     }
     pool_free(tmp);
-    if (rc) {
-        del_buf(*out);
-        *out = nullptr;
-    }
-    return rc;
+    return keep_out(rc, out);
 }
 
 int scry_hip_matmul_strided_batched(scry_buf a, scry_buf b, int batch, int m, int k, int n,
@@ -755,7 +756,8 @@ int scry_hip_matmul_strided_batched(scry_buf a, scry_buf b, int batch, int m, in
     if (a->n < (size_t)batch * m * k || b->n < (size_t)batch * k * n)
         return set_error(SCRY_ERR_INVALID, "matmul_strided_batched: operand too short");
     SCRY_TRY(new_buf((size_t)batch * m * n, out));
-    return launch_matmul_f32(a->d, b->d, batch, m, k, n, trans_a, trans_b, nullptr, (*out)->d, ctx().stream);
+    return keep_out(launch_matmul_f32(a->d, b->d, batch, m, k, n, trans_a, trans_b, nullptr, (*out)->d, ctx().stream),
+                    out);
 }
 
 int scry_hip_rmsnorm(scry_buf x, scry_buf w, int rows, int d, float eps, scry_buf *out) {

@@ -1,5 +1,6 @@
 """Where the device has no memory left for a workspace the work runs without
-it (host logic, on a runtime without a device)."""
+it, and an op that fails leaves no output (host logic, on a runtime without a
+device)."""
 import pytest
 
 OPS = """
@@ -37,4 +38,18 @@ F.fake_limit(used + (1 << 20 if {op!r} == "few_rows" else 5 << 20))  # activatio
 assert not split(op)
 F.fake_limit(1 << 40)
 assert split(op)  # and with room again
+""")
+
+
+@pytest.mark.parametrize("call", ["matmul(A.h, W.h, 64, 4096, 4096, 0, 0", "matmul_bias(A.h, W.h, A.h, 64, 4096, 4096, 0, 0",
+                                  "matmul_strided_batched(A.h, W.h, 1, 64, 4096, 4096, 0, 0"])
+def test_failed_op_leaves_no_output(fake_hip, call):
+    """The launch is refused (here by a grid the runtime does not take)."""
+    fake_hip(OPS + f"""
+from esolearn_amd._lib import load
+out = C.c_void_p()
+F.fake_refuse(1)
+rc = load().scry_hip_{call}, C.byref(out))
+F.fake_refuse(0)
+assert rc != 0 and not out.value, (rc, out)
 """)

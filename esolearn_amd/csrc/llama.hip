@@ -873,6 +873,14 @@ int prefill_core(scry_llama m, scry_kv_cache *cs, int n_seq, const int64_t *toke
         g.m = n_seq;
         g.y = last_logits;
         g.ldy = m->V;
+        // int8 rows take the op-level matmul's route (4 rows x 128256 columns:
+        // 229 us as a GEMV over 4 rows) where its workspace can be had; the
+        // GEMV needs none
+        void *ws = nullptr;
+        if (!m->lm.bf16 && skinny_route(n_seq, m->h, m->lm.rows)) {
+            const int rc = ctx_workspace(skinny_ws_bytes(n_seq, m->h, m->lm.rows), &ws);
+            if (rc && rc != SCRY_ERR_OOM) return rc;
+        }
         if (m->lm.bf16) {  // the bf16 GEMV takes one activation row per launch
             g.m = 1;
             for (int i = 0; i < n_seq; i++) {
@@ -880,11 +888,7 @@ int prefill_core(scry_llama m, scry_kv_cache *cs, int n_seq, const int64_t *toke
                 g.y = last_logits + (size_t)i * m->V;
                 SCRY_TRY(launch_qgemv(EPI_STORE, g, s));
             }
-        } else if (skinny_route(n_seq, m->h, m->lm.rows)) {
-            // the op-level matmul's route: several rows on the matrix cores (4
-            // rows x 128256 columns: 229 us as a GEMV over 4 rows)
-            void *ws = nullptr;
-            SCRY_TRY(ctx_workspace(skinny_ws_bytes(n_seq, m->h, m->lm.rows), &ws));
+        } else if (ws) {
             SkinnyMM sm;
             sm.w = &m->lm;
             sm.x = P.xl;

@@ -8,11 +8,13 @@
 // layer 6.5 of 7.4 ms.
 //
 // All op work runs on the context's one stream, so a block freed by the host
-// is handed to a later op in stream order without waiting.  Blocks are filed
-// by size class (8 per power of two) under the API lock.  The cache is
-// bounded (kPoolCap) and given back when a block would exceed the bound, when
-// the device runs out of memory (dev_alloc retries) and at shutdown; blocks
-// of another device are never reused.
+// is handed to a later op in stream order without waiting.  Blocks up to
+// kPoolMax are filed by size class (8 per power of two) under the API lock;
+// larger ones, and blocks whose class finds no memory, are allocated at their
+// exact size and not kept.  The cache is bounded (kPoolCap) and given back when
+// a block would exceed the bound, when the device runs out of memory (dev_alloc
+// retries) and at shutdown; blocks of another device are never reused.
+#include <new>
 #include <unordered_map>
 
 #include "internal.h"
@@ -21,6 +23,7 @@ namespace scry {
 namespace {
 
 constexpr size_t kPoolCap = (size_t)2 << 30;  // under 1% of the card's memory
+constexpr size_t kPoolMax = kPoolCap / 2;
 
 struct Block {
     int cls, device;
@@ -61,6 +64,7 @@ void pool_trim() {
 int pool_alloc(void **p, size_t bytes) {
     std::lock_guard<std::recursive_mutex> lock(api_mutex());
     *p = nullptr;
+    if (bytes > kPoolMax) return dev_alloc(p, bytes);
     Pool &P = pool();
     const int c = class_of(bytes);
     auto it = P.free_lists.find(c);
@@ -70,8 +74,13 @@ int pool_alloc(void **p, size_t bytes) {
         P.cached -= class_bytes(c);
         return SCRY_OK;
     }
-    SCRY_TRY(dev_alloc(p, class_bytes(c)));
-    P.blocks[*p] = Block{c, ctx().device};
+    const int rc = dev_alloc(p, class_bytes(c));
+    if (rc == SCRY_ERR_OOM) return dev_alloc(p, bytes);
+    if (rc) return rc;
+    try {
+        P.blocks[*p] = Block{c, ctx().device};
+    } catch (const std::bad_alloc &) {  // not filed: freed as it is
+    }
     return SCRY_OK;
 }
 
@@ -80,16 +89,20 @@ void pool_free(void *p) {
     std::lock_guard<std::recursive_mutex> lock(api_mutex());
     Pool &P = pool();
     auto it = P.blocks.find(p);
-    const size_t n = it == P.blocks.end() ? 0 : class_bytes(it->second.cls);
-    if (n == 0 || !ctx().init || it->second.device != ctx().device || n > kPoolCap / 2) {
-        if (n) P.blocks.erase(it);
-        if (ctx().init) (void)hipStreamSynchronize(ctx().stream);
-        dev_free(p);
-        return;
+    if (it != P.blocks.end() && ctx().init && it->second.device == ctx().device) {
+        const int c = it->second.cls;
+        const size_t n = class_bytes(c);
+        if (P.cached + n > kPoolCap) pool_trim();
+        try {
+            P.free_lists[c].push_back(p);
+            P.cached += n;
+            return;
+        } catch (const std::bad_alloc &) {
+        }
     }
-    if (P.cached + n > kPoolCap) pool_trim();
-    P.free_lists[it->second.cls].push_back(p);
-    P.cached += n;
+    if (it != P.blocks.end()) P.blocks.erase(it);
+    if (ctx().init) (void)hipStreamSynchronize(ctx().stream);
+    dev_free(p);
 }
 
 }  // namespace scry

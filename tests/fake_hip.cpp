@@ -66,7 +66,7 @@ const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "success"
 hipError_t hipMalloc(void **p, size_t n) {
     State &s = S();
     *p = nullptr;
-    if (s.used > s.limit || n > s.limit - s.used) return hipErrorOutOfMemory;
+    if (n >> 46 || s.used > s.limit || n > s.limit - s.used) return hipErrorOutOfMemory;
     void *q = mmap(nullptr, n + 4096, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     if (q == MAP_FAILED) return hipErrorOutOfMemory;
     s.blocks[q] = n;

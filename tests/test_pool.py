@@ -1,0 +1,48 @@
+"""The storage pool's bound, its sizes and what it gives back (host logic, on a
+runtime without a device).  Sizes in f32 values."""
+
+
+def test_cached_blocks_are_given_back_for_an_allocation(fake_hip):
+    fake_hip("""
+s = [B.zeros(1 << 26) for _ in range(4)]  # 1 GB
+used = F.fake_used()
+F.fake_limit(used)
+for b in s: b.free()
+assert F.fake_used() == used
+x = B.zeros(200 << 20)  # 800 MB: only without the cache
+assert F.fake_used() < used
+""")
+
+
+def test_large_blocks_have_their_exact_size(fake_hip):
+    fake_hip("""
+used = F.fake_used()
+n = (1 << 28) + 3
+x = B.zeros(n)
+assert F.fake_used() - used == 4 * n
+x.free()
+assert F.fake_used() == used
+""")
+
+
+def test_a_size_that_fits_exactly(fake_hip):
+    fake_hip("""
+n = (1 << 26) + 3  # its class has 32 MB more
+F.fake_limit(F.fake_used() + 4 * n)
+x = B.zeros(n)
+used = F.fake_used()
+x.free()
+assert F.fake_used() == used - 4 * n  # not kept under a class it is too small for
+""")
+
+
+def test_sizes_beyond_any_device_are_refused(fake_hip):
+    fake_hip("""
+for n in ((1 << 62) - 1, (1 << 61) + (1 << 60) + 1, 1 << 50):
+    try:
+        B.zeros(n)
+    except E.ScryHipError as e:
+        assert e.code == 3
+    else:
+        raise SystemExit(f"{n} values were accepted")
+""")

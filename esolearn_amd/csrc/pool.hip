@@ -11,9 +11,11 @@
 // is handed to a later op in stream order without waiting.  Blocks up to
 // kPoolMax are filed by size class (8 per power of two) under the API lock;
 // larger ones, and blocks whose class finds no memory, are allocated at their
-// exact size and not kept.  The cache is bounded (kPoolCap) and given back when
-// a block would exceed the bound, when the device runs out of memory (dev_alloc
-// retries) and at shutdown; blocks of another device are never reused.
+// exact size and not kept.  The cache is bounded (kPoolCap: the largest blocks
+// are given back first) and given back whole when the device runs out of memory
+// (dev_alloc retries) and at shutdown; blocks of another device are never
+// reused.
+#include <map>
 #include <new>
 #include <unordered_map>
 
@@ -30,7 +32,7 @@ struct Block {
 };
 struct Pool {
     std::unordered_map<void *, Block> blocks;  // every live or cached block
-    std::unordered_map<int, std::vector<void *>> free_lists;
+    std::map<int, std::vector<void *>> free_lists;
     size_t cached = 0;
 };
 Pool &pool() {
@@ -92,7 +94,14 @@ void pool_free(void *p) {
     if (it != P.blocks.end() && ctx().init && it->second.device == ctx().device) {
         const int c = it->second.cls;
         const size_t n = class_bytes(c);
-        if (P.cached + n > kPoolCap) pool_trim();
+        for (auto l = P.free_lists.rbegin(); P.cached + n > kPoolCap && l != P.free_lists.rend(); ++l)
+            while (P.cached + n > kPoolCap && !l->second.empty()) {
+                void *q = l->second.back();
+                l->second.pop_back();
+                P.cached -= class_bytes(l->first);
+                P.blocks.erase(q);
+                dev_free(q);  // waits for the work that still uses it
+            }
         try {
             P.free_lists[c].push_back(p);
             P.cached += n;

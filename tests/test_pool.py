@@ -2,6 +2,23 @@
 runtime without a device).  Sizes in f32 values."""
 
 
+def test_cache_is_bounded_and_keeps_small_blocks(fake_hip):
+    fake_hip("""
+small = [B.zeros(1000 + 100 * i) for i in range(20)]
+big = [B.zeros(1 << 27) for _ in range(6)]  # 512 MB each
+live = F.fake_used()
+for s in small: s.free()
+for s in big: s.free()
+assert F.fake_used() <= 2 << 30 and F.fake_used() > 1 << 30
+n = F.fake_mallocs()
+again = [B.zeros(1000 + 100 * i) for i in range(20)] + [B.zeros(1 << 27) for _ in range(3)]
+assert F.fake_mallocs() == n
+from esolearn_amd._lib import call
+call("scry_hip_shutdown")
+assert F.fake_used() < (3 << 29) + (1 << 20)  # the live storage
+""")
+
+
 def test_cached_blocks_are_given_back_for_an_allocation(fake_hip):
     fake_hip("""
 s = [B.zeros(1 << 26) for _ in range(4)]  # 1 GB

@@ -42,7 +42,7 @@ import esolearn_amd as E
 F = C.CDLL(sys.argv[1])
 F.fake_used.restype = C.c_size_t
 F.fake_limit.argtypes = [C.c_size_t]
-F.fake_launches.restype = C.c_char_p
+F.fake_launches.restype = F.fake_kernels.restype = C.c_char_p
 def launches():
     return F.fake_launches().decode().splitlines()
 E.init(0)

@@ -38,6 +38,13 @@ long fake_mallocs() { return S().mallocs; }
 long fake_frees() { return S().frees; }
 void fake_limit(size_t bytes) { S().limit = bytes; }
 void fake_copies(int on) { S().copies = on != 0; }
+// mangled names of every kernel in the library, a line each
+const char *fake_kernels() {
+    static std::string all;
+    all.clear();
+    for (auto &k : S().kernels) all += k.second + "\n";
+    return all.c_str();
+}
 void fake_refuse(int on) { S().refuse = on != 0; }  // launches fail
 // "mangled kernel name, grid x y z" lines since the last call
 const char *fake_launches() {

@@ -1,7 +1,7 @@
-"""The digit GEMM's tiles and k splits (matmul_i8_f32 above 16 rows, the int8
-model's prefill): small integer activations have exact digit planes, so every
-tile and split must give the exact integer sums; and a model whose prefill
-GEMMs split k against its token-by-token decode."""
+"""The GEMMs' tiles and k splits (matmul_i8_f32 and bf16 matmul above 16 rows,
+prefill): with integer operands every tile and split must give the exact sums;
+prefill's residual and SwiGLU epilogues against the token-by-token decode.
+test_gemm_tiles_covered.py holds that the shapes here reach every tile."""
 import numpy as np
 import pytest
 
@@ -13,7 +13,8 @@ F = np.float32
     (17, 64, 5), (33, 100, 131), (32, 2048, 128), (37, 4096, 260), (64, 768, 768), (65, 3072, 770),
     (130, 4096, 1030), (200, 768, 2304), (129, 8192, 4096), (300, 1024, 4097), (512, 2048, 2050),
     (129, 256, 28416), (600, 128, 28000), (255, 192, 21889), (1100, 64, 13000),
-    (384, 1100, 22018), (600, 1024, 14339), (1500, 1024, 6145), (511, 2048, 22013)])
+    (384, 1100, 22018), (600, 1024, 14339), (1500, 1024, 6145), (511, 2048, 22013),
+    (174, 40, 11339), (77, 6434, 5879), (1416, 51, 681), (1183, 1997, 5), (293, 3552, 6531)])
 def test_exact_sums(hip, m, k, n):
     print(f"[case] {m} x {k} x {n}", flush=True)
     B = hip.HipBackend
@@ -84,7 +85,8 @@ def test_prefill_in_two_launches_matches_shorter(hip, mode, seq, ffn):
 
 @pytest.mark.parametrize("m,k,n", [
     (17, 64, 5), (37, 100, 131), (32, 4096, 260), (64, 768, 768), (130, 4096, 1030), (200, 3072, 770),
-    (129, 1280, 5120), (300, 1024, 4097), (512, 8192, 1024), (600, 2048, 14339)])
+    (129, 1280, 5120), (300, 1024, 4097), (512, 8192, 1024), (600, 2048, 14339),
+    (174, 40, 11339), (67, 4864, 2815), (22, 47, 16838), (17, 2240, 2559), (178, 5451, 11150)])
 def test_bf16_exact_sums(hip, m, k, n):
     """The bf16 GEMM's tiles and splits: integers exact in bf16, sums exact in f32."""
     print(f"[case] bf16 {m} x {k} x {n}", flush=True)
@@ -122,7 +124,8 @@ def test_bf16_prefill_small_tiles_match_decode(hip, seq):
 
 @pytest.mark.parametrize("m,k,n", [
     (17, 64, 5), (33, 100, 131), (40, 4096, 260), (64, 768, 768), (130, 3000, 1030), (129, 4096, 4096),
-    (300, 1024, 4097), (512, 11008, 516), (600, 1024, 14339)])
+    (300, 1024, 4097), (512, 11008, 516), (600, 1024, 14339),
+    (174, 40, 11339), (1416, 51, 681), (1183, 1997, 5), (695, 2946, 6226)])
 def test_block32_exact_sums(hip, m, k, n):
     """Block-32 scales that are powers of two: every product and sum is exact in f32."""
     print(f"[case] block32 {m} x {k} x {n}", flush=True)
@@ -151,3 +154,77 @@ def test_block32_prefill_matches_decode(hip, seq):
         ref, _ = m.forward_with_llama_cache(int(t), p, cd)
     assert np.abs(last - ref).max() <= 1e-3 * np.abs(ref).max()
     m.free()
+
+
+PREFILL_SHAPES = [  # weights, hidden, ffn, prompt
+    ("per_tensor", 128, 370, 21), ("per_tensor", 1024, 128, 19), ("per_tensor", 2560, 1152, 36), ("per_tensor", 128, 1152, 583),
+    ("per_tensor", 128, 4800, 210), ("per_tensor", 128, 4800, 456), ("per_tensor", 2560, 104, 842), ("per_tensor", 640, 8704, 886),
+    ("per_tensor", 2176, 8910, 117), ("per_tensor", 3072, 126, 333), ("per_tensor", 2944, 260, 394),
+    ("per_tensor", 1216, 62, 804), ("per_tensor", 4096, 2730, 2040),
+    ("block32", 128, 370, 26), ("block32", 128, 862, 20), ("block32", 2560, 104, 45), ("block32", 2432, 110, 125),
+    ("block32", 128, 4800, 303), ("block32", 128, 3546, 139), ("block32", 384, 2324, 420), ("block32", 384, 2324, 1279),
+    ("block32", 2432, 110, 510), ("block32", 2432, 110, 1140), ("block32", 4224, 2046, 34), ("block32", 4096, 512, 2040),
+    ("bf16", 128, 448, 19), ("bf16", 128, 1152, 26), ("bf16", 2560, 104, 17), ("bf16", 2432, 110, 39), ("bf16", 128, 862, 615),
+    ("bf16", 128, 4800, 88), ("bf16", 256, 1758, 707), ("bf16", 2432, 110, 391), ("bf16", 2560, 104, 413), ("bf16", 2816, 426, 169),
+    ("bf16", 2688, 142, 934), ("bf16", 128, 4800, 649), ("bf16", 4096, 512, 2040),
+]
+
+
+def prefill_model(E, mode, h, ffn, seq):
+    import esolearn_amd.llama as EL
+    q = {"per_tensor": EL.QUANT_PER_TENSOR, "block32": EL.QUANT_BLOCK32, "bf16": EL.QUANT_BF16}[mode]
+    nh = h // (64 if h % 128 else 128)
+    cfg = E.LlamaConfig(vocab_size=96, hidden_size=h, intermediate_size=ffn, n_layers=2, n_heads=nh,
+                        n_kv_heads=nh if nh % 2 else nh // 2, max_seq_len=2048, rope_theta=10000.0,
+                        tie_word_embeddings=False)
+    return E.LlamaModel.new_random(cfg, 3, quant_mode=q, init_on_device=True)
+
+
+@pytest.mark.parametrize("mode,h,ffn,seq", PREFILL_SHAPES)
+def test_prefill_rows_match_decode(hip, mode, h, ffn, seq):
+    """Every row of the second layer's K and V (the first layer's residual and
+    SwiGLU epilogues, all columns mixed by K's and V's products) against the
+    decode path.  Per row, relative in 2-norm: 1e-3 as the other prefill tests;
+    bf16: in each of the four products of a layer a value may round to the other
+    neighbour, 2^-8 of it, in quadrature 8e-3.  One wrong column would be 1 /
+    sqrt(columns), 1e-2 or more."""
+    print(f"[case] {mode} h={h} ffn={ffn} seq={seq}", flush=True)
+    m = prefill_model(hip, mode, h, ffn, seq)
+    toks = np.random.default_rng(seq).integers(0, 96, seq)
+    cp, cd = m.new_llama_kv_cache(seq), m.new_llama_kv_cache(seq)
+    m.prefill([cp], toks[None, :])
+    for p, t in enumerate(toks):
+        m.forward_with_llama_cache(int(t), p, cd)
+    for a, b in zip(cp.layer(1), cd.layer(1)):
+        a, b = a.reshape(seq, -1).astype(np.float64), b.reshape(seq, -1).astype(np.float64)
+        err = np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1)
+        print(f"[err] {err.max():.2e}", flush=True)
+        assert err.max() <= (8e-3 if mode == "bf16" else 1e-3)
+    m.free()
+
+
+@pytest.mark.parametrize("kind", ["bf16", "block32", "per_tensor"])
+def test_planes_above_2_gib(hip, kind):
+    """More activation bytes than a buffer resource reaches: the register-staged
+    kernel (per_tensor: only k above the digit kernel's)."""
+    print(f"[case] {kind}", flush=True)
+    B = hip.HipBackend
+    rows, reps, n = 513, 256, 70
+    k = 16448 if kind == "per_tensor" else 8224
+    m = rows * reps if kind != "per_tensor" else rows * reps // 2
+    rng = np.random.default_rng(k)
+    a = rng.integers(-3, 4, (rows, k)).astype(F)
+    q = rng.integers(-40, 41, (k, n)).astype(np.int8)
+    A = B.repeat_kv(B.from_vec(a), 1, m // rows, rows, k)  # the rows again and again
+    if kind == "bf16":
+        B.set_bf16_mode(True)
+        try:
+            c = B.matmul(A, B.from_vec(q.astype(F)), m, k, n)
+        finally:
+            B.set_bf16_mode(False)
+    elif kind == "block32":
+        c = B.matmul_i8_f32_block32(A, B.i8_from_vec(q), B.ones(n * ((k + 31) // 32)), m, k, n)
+    else:
+        c = B.matmul_i8_f32(A, B.i8_from_vec(q), 1.0, m, k, n)
+    ref = (a.astype(np.float64) @ q.astype(np.float64)).astype(F)  # below 2^24: exact
+    assert np.array_equal(c.to_vec().reshape(-1, rows, n), np.broadcast_to(ref, (m // rows, rows, n)))

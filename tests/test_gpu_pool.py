@@ -26,24 +26,39 @@ def test_reuse_while_queued(hip):
     assert np.array_equal(s.to_vec(), ref)
 
 
-@pytest.mark.parametrize("m,k,n", [(20, 100, 64), (150, 768, 96)])
-def test_results_do_not_depend_on_old_contents(hip, m, k, n):
-    """The GEMM planes come from reused blocks: fill such blocks with NaN and
-    infinities first (rows past m and columns past k are theirs)."""
+def _dirty(B, value):
+    """Two free blocks of every size class up to 2 MB ((8 + i) << (e + 5) bytes) that hold `value`."""
+    junk = [B.from_vec(np.full((8 + i) << (e + 3), value, F)) for e in range(14) for i in range(8) for _ in range(2)]
+    for j in junk:
+        j.free()
+
+
+@pytest.mark.parametrize("m,k,n", [(20, 100, 64), (150, 768, 96), (150, 700, 33)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_results_do_not_depend_on_old_contents(hip, m, k, n, bad):
+    """The GEMM planes come from reused blocks and are not cleared: rows past m
+    and columns past k are what the block held.  Every block a call can get holds
+    NaN or infinities first; integer operands, so the results are exact."""
+    print(f"[case] {m} x {k} x {n} {bad}", flush=True)
     B = hip.HipBackend
     rng = np.random.default_rng(m)
-    a = rng.normal(size=(m, k)).astype(F)
-    q = rng.integers(-127, 128, (k, n)).astype(np.int8)
-    A, W = B.from_vec(a), B.i8_from_vec(q)
-    sc = B.from_vec(np.ones(n * ((k + 31) // 32), F))
-    ref = [B.matmul_i8_f32(A, W, 0.1, m, k, n).to_vec(), B.matmul_i8_f32_block32(A, W, sc, m, k, n).to_vec()]
-    for bad in (np.nan, np.inf):
-        junk = [B.from_vec(np.full(1 << e, bad, F)) for e in range(8, 20) for _ in range(2)]
-        junk += [B.from_vec(np.full(3 << e, bad, F)) for e in range(8, 20)]
-        for j in junk:
-            j.free()
-        assert np.array_equal(B.matmul_i8_f32(A, W, 0.1, m, k, n).to_vec(), ref[0])
-        assert np.array_equal(B.matmul_i8_f32_block32(A, W, sc, m, k, n).to_vec(), ref[1])
+    a = rng.integers(-8, 9, (m, k)).astype(F)
+    q = rng.integers(-60, 61, (k, n)).astype(np.int8)
+    ref = a.astype(np.float64) @ q.astype(np.float64)
+    A, W, Wf, sc = B.from_vec(a), B.i8_from_vec(q), B.from_vec(q.astype(F)), B.ones(n * ((k + 31) // 32))
+
+    def bf16():
+        B.set_bf16_mode(True)
+        try:
+            return B.matmul(A, Wf, m, k, n)
+        finally:
+            B.set_bf16_mode(False)
+
+    for op in (lambda: B.matmul_i8_f32(A, W, 1.0, m, k, n), lambda: B.matmul_i8_f32_block32(A, W, sc, m, k, n), bf16,
+               lambda: B.matmul(A, Wf, m, k, n)):
+        for _ in range(2):
+            _dirty(B, bad)
+            assert np.array_equal(op().to_vec().reshape(m, n), ref)
 
 
 def test_threads(hip):

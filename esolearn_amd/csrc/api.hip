@@ -1164,7 +1164,7 @@ int scry_hip_rope(scry_buf x, size_t rows, int last_dim, int pos, int head_dim, 
                                       ctx().stream);
         rc = e == hipSuccess ? SCRY_OK : hip_fail(e, "rope table upload", __FILE__, __LINE__);
         if (!rc) rc = launch_rope_row(x->d, rows, last_dim, head_dim, d_cs, (*out)->d, ctx().stream);
-        if (!rc) rc = sync();  // the table is freed below
+        if (!rc) rc = sync();  // the upload reads the host table
     }
     pool_free(d_cs);
     return rc;

@@ -39,8 +39,9 @@ struct MMArgs {
 // requested before the current step's MFMAs and written to the other LDS
 // buffer after them (one barrier per step).
 // Measured against one thread per output with a serial f64 loop: 1500 x 1280
-// x 5120 (k in the middle) 368 us, 53 TFLOP/s, against about 10 ms; attention
-// scores 20 x [1500 x 64] x [64 x 1500] 134 us against 2.7 ms, values 123 us.
+// x 5120 (k in the middle) 341-368 us (two cards), 53-58 TFLOP/s, against about
+// 10 ms; attention scores 20 x [1500 x 64] x [64 x 1500] 122-134 us against 2.7
+// ms, values 111-123 us with k_mm_reduce.
 constexpr int MM_T = 256, MM_BK = 32, MM_S = 36;
 
 // KC: the operand is stored k-contiguous ([row][k], ld = k), else [k][row]

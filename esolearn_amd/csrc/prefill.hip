@@ -690,7 +690,7 @@ __global__ __launch_bounds__(G_THREADS, B32 ? 1 : 2) void k_gemm(GemmP p) {
 // WBF: bf16 weight rows (128 B per column and step, read as they are) and one
 // activation plane (the bf16 model); else int8 weights and hi, lo planes.
 // The bf16 model's short prompts and the op-level bf16 matmul also take
-// smaller tiles and k splits (pick_ring): with 128 x 256, 37 rows x 4096
+// smaller tiles and k splits (pick_tile, pick_cut): with 128 x 256, 37 rows x 4096
 // columns are 16 workgroups.  Without splits a tile changes no bit (the k
 // order is the same); a split's f32 sums are added in split order.
 // B32: int8 weights with block-32 scales: the two scales a step has per column

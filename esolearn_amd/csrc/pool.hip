@@ -11,11 +11,11 @@
 // is handed to a later op in stream order without waiting.  Blocks up to
 // kPoolMax are filed by size class (8 per power of two) under the API lock;
 // larger ones, and blocks whose class finds no memory, are allocated at their
-// exact size and not kept.  The cache is bounded (kPoolCap: the largest blocks
-// are given back first) and given back whole when the device runs out of memory
-// (dev_alloc retries) and at shutdown; blocks of another device are never
+// exact size and not kept.  The cache is bounded (kPoolCap: the blocks unused for
+// longest are given back first, so that what a program no longer needs does not
+// push out what it uses) and given back whole when the device runs out of
+// memory (dev_alloc retries) and at shutdown; blocks of another device are never
 // reused.
-#include <map>
 #include <new>
 #include <unordered_map>
 
@@ -30,10 +30,15 @@ constexpr size_t kPoolMax = kPoolCap / 2;
 struct Block {
     int cls, device;
 };
+struct Free {
+    void *p;
+    uint64_t when;  // number of the free
+};
 struct Pool {
     std::unordered_map<void *, Block> blocks;  // every live or cached block
-    std::map<int, std::vector<void *>> free_lists;
+    std::unordered_map<int, std::vector<Free>> free_lists;  // by class, oldest first
     size_t cached = 0;
+    uint64_t frees = 0;
 };
 Pool &pool() {
     static Pool *p = new Pool;  // never destroyed: storage may be freed during process exit
@@ -49,15 +54,27 @@ int class_of(size_t bytes) {
     return 8 * e + (int)((bytes - 1) >> (e + 5)) - 8 + 1;
 }
 
+// (P.cached > 0)
+void give_back_oldest(Pool &P) {
+    auto old = P.free_lists.end();
+    for (auto l = P.free_lists.begin(); l != P.free_lists.end(); ++l)
+        if (!l->second.empty() && (old == P.free_lists.end() || l->second[0].when < old->second[0].when)) old = l;
+    void *p = old->second[0].p;
+    old->second.erase(old->second.begin());
+    P.cached -= class_bytes(old->first);
+    P.blocks.erase(p);
+    dev_free(p);  // waits for the work that still uses it
+}
+
 }  // namespace
 
 void pool_trim() {
     std::lock_guard<std::recursive_mutex> lock(api_mutex());
     Pool &P = pool();
     for (auto &l : P.free_lists)
-        for (void *p : l.second) {
-            P.blocks.erase(p);
-            (void)hipFree(p);  // waits for the work that still uses it
+        for (const Free &f : l.second) {
+            P.blocks.erase(f.p);
+            dev_free(f.p);  // waits for the work that still uses it
         }
     P.free_lists.clear();
     P.cached = 0;
@@ -71,7 +88,7 @@ int pool_alloc(void **p, size_t bytes) {
     const int c = class_of(bytes);
     auto it = P.free_lists.find(c);
     if (it != P.free_lists.end() && !it->second.empty()) {
-        *p = it->second.back();
+        *p = it->second.back().p;
         it->second.pop_back();
         P.cached -= class_bytes(c);
         return SCRY_OK;
@@ -94,16 +111,9 @@ void pool_free(void *p) {
     if (it != P.blocks.end() && ctx().init && it->second.device == ctx().device) {
         const int c = it->second.cls;
         const size_t n = class_bytes(c);
-        for (auto l = P.free_lists.rbegin(); P.cached + n > kPoolCap && l != P.free_lists.rend(); ++l)
-            while (P.cached + n > kPoolCap && !l->second.empty()) {
-                void *q = l->second.back();
-                l->second.pop_back();
-                P.cached -= class_bytes(l->first);
-                P.blocks.erase(q);
-                dev_free(q);  // waits for the work that still uses it
-            }
+        while (P.cached + n > kPoolCap) give_back_oldest(P);
         try {
-            P.free_lists[c].push_back(p);
+            P.free_lists[c].push_back(Free{p, P.frees++});
             P.cached += n;
             return;
         } catch (const std::bad_alloc &) {

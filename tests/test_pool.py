@@ -2,13 +2,13 @@
 runtime without a device).  Sizes in f32 values."""
 
 
-def test_cache_is_bounded_and_keeps_small_blocks(fake_hip):
+def test_cache_is_bounded_and_keeps_the_last_freed(fake_hip):
     fake_hip("""
 small = [B.zeros(1000 + 100 * i) for i in range(20)]
 big = [B.zeros(1 << 27) for _ in range(6)]  # 512 MB each
 live = F.fake_used()
-for s in small: s.free()
 for s in big: s.free()
+for s in small: s.free()
 assert F.fake_used() <= 2 << 30 and F.fake_used() > 1 << 30
 n = F.fake_mallocs()
 again = [B.zeros(1000 + 100 * i) for i in range(20)] + [B.zeros(1 << 27) for _ in range(3)]
@@ -16,6 +16,19 @@ assert F.fake_mallocs() == n
 from esolearn_amd._lib import call
 call("scry_hip_shutdown")
 assert F.fake_used() < (3 << 29) + (1 << 20)  # the live storage
+""")
+
+
+def test_cache_full_of_blocks_no_longer_used(fake_hip):
+    """They make room for the blocks in use, which then stay."""
+    fake_hip("""
+old = [B.zeros(75 << 20) for _ in range(6)] + [B.zeros(1000 + i) for i in range(300)]  # 6 x 300 MB
+for s in old: s.free()
+for step in range(4):
+    n = F.fake_mallocs()
+    s = [B.zeros(1 << 27) for _ in range(3)]
+    for x in s: x.free()
+    assert step < 2 or F.fake_mallocs() == n, step
 """)
 
 

@@ -95,8 +95,11 @@ __global__ void k_rope(const float *__restrict__ x, int seq, int n_heads, int hd
         const float c = (float)cos(ang), sn = (float)sin(ang);
 #pragma unroll
         for (int h = 0; h < ROPE_H; h++) {
-            float r0 = __fsub_rn(__fmul_rn(v[h].x, c), __fmul_rn(v[h].y, sn));
-            float r1 = __fadd_rn(__fmul_rn(v[h].x, sn), __fmul_rn(v[h].y, c));
+            // the cosine products are fused, as written: of products left to the
+            // compiler it fused either, depending on the code around them, and
+            // the last bit with it
+            float r0 = fmaf(v[h].x, c, -__fmul_rn(v[h].y, sn));
+            float r1 = fmaf(v[h].y, c, __fmul_rn(v[h].x, sn));
             if (scaled) {
                 r0 = __fmul_rn(r0, scale);
                 r1 = __fmul_rn(r1, scale);

@@ -115,3 +115,23 @@ def test_argmax_ranges(hip, n):
         tail = x[n // 2 + 2:]
         want = n // 2 + 2 + (len(tail) - 1 - int(tail[::-1].argmax())) if len(tail) else n // 2 + 1
         assert B.argmax(B.from_vec(x)) == want
+
+
+@pytest.mark.parametrize("s,nh,hd,pos", [(1, 32, 128, 1000), (37, 9, 64, 0), (5, 1, 2, 3)])
+def test_rope_fused_products(hip, s, nh, hd, pos):
+    """Which product of a rotated pair is rounded by itself: the sine's, both for
+    the even and the odd value (the other way about a sixth of the values differ
+    in their last bit).  The products are exact in 64-bit significands and the
+    sums nearly always; cos and sin are f64 rounded to f32, by another library."""
+    B = hip.HipBackend
+    rng = np.random.default_rng(s + nh)
+    x = rng.normal(size=(s, nh, hd // 2, 2)).astype(F)
+    f = (1.0 / 10000.0 ** (2.0 * np.arange(hd // 2) / hd)).astype(F)
+    ang = (pos + np.arange(s, dtype=np.float64))[:, None, None] * f.astype(np.float64)
+    c, sn = np.cos(ang).astype(F), np.sin(ang).astype(F)
+    L = np.longdouble
+    ref = np.stack([(L(1) * x[..., 0] * c - x[..., 1] * sn).astype(F), (L(1) * x[..., 1] * c + x[..., 0] * sn).astype(F)], -1)
+    got = B.rope_with_freqs_preloaded(B.from_vec(x.ravel()), s, nh, hd, pos, B.from_vec(f)).to_vec().reshape(x.shape)
+    scaled = B.rope_with_freqs_scaled_preloaded(B.from_vec(x.ravel()), s, nh, hd, pos, B.from_vec(f), 0.125).to_vec()
+    assert (got != ref).mean() <= 1e-3
+    assert np.array_equal(scaled, (got * F(0.125)).ravel())

@@ -142,6 +142,13 @@ __global__ void k_scale(const float *__restrict__ x, size_t n, float s, float *_
     });
 }
 
+// x * scale rounded to f32: a product that may be contracted (as __fmul_rn's
+// may) is fused into the subtraction of the maximum
+__device__ __forceinline__ float scaled_value(float x, float scale) {
+#pragma clang fp contract(off)
+    return x * scale;
+}
+
 // softmax (cpu.rs:336-366) and scaled_softmax (cpu.rs:300-334): v = x or x *
 // scale (f32), f32 max (NaN ignored), e = expf(v - max) kept as f32, f64 sum,
 // out = f32(f64(e) * (1 / sum)) (within an f64 ulp of e / sum: the f64 divide
@@ -167,7 +174,7 @@ __global__ __launch_bounds__(256) void k_softmax_reg(const float *__restrict__ x
     }
 #pragma unroll
     for (int c = 0; c < NV; c++) {
-        if (SCALED && c * W + t < cols) v[c] = __fmul_rn(v[c], scale);
+        if (SCALED && c * W + t < cols) v[c] = scaled_value(v[c], scale);
         mx = fmaxf(mx, v[c]);
     }
 #pragma unroll
@@ -208,14 +215,14 @@ __global__ __launch_bounds__(256) void k_softmax(const float *__restrict__ x, in
     __shared__ float redf[4];
     __shared__ double redd[4];
     float mx = -INFINITY;
-    for (int j = threadIdx.x; j < cols; j += 256) mx = fmaxf(mx, SCALED ? __fmul_rn(r[j], scale) : r[j]);
+    for (int j = threadIdx.x; j < cols; j += 256) mx = fmaxf(mx, SCALED ? scaled_value(r[j], scale) : r[j]);
     for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     if ((threadIdx.x & 63) == 0) redf[threadIdx.x >> 6] = mx;
     __syncthreads();
     mx = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
     double sum = 0.0;
     for (int j = threadIdx.x; j < cols; j += 256) {
-        const float e = expf(__fsub_rn(SCALED ? __fmul_rn(r[j], scale) : r[j], mx));
+        const float e = expf(__fsub_rn(SCALED ? scaled_value(r[j], scale) : r[j], mx));
         o[j] = e;
         sum += (double)e;
     }

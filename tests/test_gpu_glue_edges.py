@@ -135,3 +135,13 @@ def test_rope_fused_products(hip, s, nh, hd, pos):
     scaled = B.rope_with_freqs_scaled_preloaded(B.from_vec(x.ravel()), s, nh, hd, pos, B.from_vec(f), 0.125).to_vec()
     assert (got != ref).mean() <= 1e-3
     assert np.array_equal(scaled, (got * F(0.125)).ravel())
+
+
+@pytest.mark.parametrize("rows,cols", [(2, 100), (1100, 513), (3, 8192), (3, 8193), (2, 20000)])
+def test_scaled_softmax_rounds_the_scaled_values(hip, rows, cols):
+    """x * scale is rounded to f32 before the maximum is taken off: the same bits
+    as softmax of the scaled values."""
+    B = hip.HipBackend
+    x = np.random.default_rng(cols).normal(0, 4, rows * cols).astype(F)
+    got = B.scaled_softmax(B.from_vec(x), 0.13, rows, cols).to_vec()
+    assert np.array_equal(got, B.softmax(B.from_vec(x * F(0.13)), rows, cols).to_vec())

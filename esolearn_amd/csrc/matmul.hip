@@ -58,17 +58,18 @@ constexpr int MM_T = 256, MM_BK = 32, MM_S = 36;
 // range (scalar instructions only: as fast as one resource and a scalar offset
 // of u rows, which the compiler leaves out of what the range check promises).
 // LD_QUAD reads 16 bytes along k (k % 4 == 0), LD_WORD single values; LD_WIDE
-// is for matrices whose offsets inside a tile do not fit 31 bits.
-enum { LD_WIDE = 0, LD_WORD = 1, LD_QUAD = 2 };
+// is for matrices whose offsets inside a tile do not fit 31 bits, LD_HUGE for
+// dimensions whose last tile or step ends past 2^31 - 1 (unsigned indexes, which
+// made LD_WIDE 5-12% slower).
+enum { LD_WIDE = 0, LD_WORD = 1, LD_QUAD = 2, LD_HUGE = 3 };
 
-// k positions, and rows and columns at a tile's end: above the LD_WIDE limit
-// they may pass 2^31 - 1
+// k positions, and rows and columns at a tile's end
 template <int LD>
 struct Index {
     typedef int T;
 };
 template <>
-struct Index<LD_WIDE> {
+struct Index<LD_HUGE> {
     typedef unsigned T;
 };
 
@@ -102,12 +103,12 @@ struct Stage {
     // MFMAs that are to hide them
     __device__ __forceinline__ void load(const float *p, int rows, int k, int r0, K k0, K kend) {
         const int left = (int)(kend - k0);
-        if (LD == LD_WIDE) {
+        if (LD == LD_WIDE || LD == LD_HUGE) {
 #pragma unroll
             for (int j = 0; j < N; j++) {
                 int row, q;
                 slot(j, row, q);
-                const unsigned r = min((unsigned)(r0 + row), (unsigned)(rows - 1));
+                const K r = min((K)r0 + row, (K)(rows - 1));
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const K c = min(k0 + 4 * q + u, (K)(k - 1));
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(256) void k_mv_rows(const float *__restrict__ a, co
         for (int i = 0; i < MT; i++) acc[r][i] = 0.0;
     constexpr int W = VEC ? 4 : 1;
 #pragma unroll 2
-    for (unsigned p = l * W; p < (unsigned)k; p += G * W) {  // unsigned: k may be 2^31 - 1
+    for (int p = l * W; p < k; p += G * W) {
         float bv[MV_R][W], av[MT][W];
 #pragma unroll
         for (int r = 0; r < MV_R; r++) {
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(256) void k_mv_rows(const float *__restrict__ a, co
 template <int MT, int W>
 __global__ __launch_bounds__(256) void k_mv_cols(const float *__restrict__ a, const float *__restrict__ b,
                                                  const float *__restrict__ bias, int batch, int m, int k, int n,
-                                                 int ta, int cg, int splits, unsigned kchunk, float *__restrict__ c,
+                                                 int ta, int cg, int splits, int kchunk, float *__restrict__ c,
                                                  double *__restrict__ part) {
     __shared__ double red[MT * W * 256];
     const int bt = blockIdx.z, sp = blockIdx.y, kg = 256 / cg;
@@ -349,18 +350,18 @@ __global__ __launch_bounds__(256) void k_mv_cols(const float *__restrict__ a, co
     const int j0 = (blockIdx.x * cg + tc) * W;
     const float *A = a + (size_t)bt * m * k;
     const float *B = b + (size_t)bt * k * n + min(j0, n - W);
-    const unsigned kb = sp * kchunk, ke = min((unsigned)k, kb + kchunk);
+    const int kb = sp * kchunk, ke = min(k, kb + kchunk);
     double acc[MT][W];
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
         for (int u = 0; u < W; u++) acc[i][u] = 0.0;
     constexpr int U = 8;  // rows in flight
-    for (unsigned p0 = kb + tk; p0 < ke; p0 += U * kg) {
+    for (int p0 = kb + tk; p0 < ke; p0 += U * kg) {
         float bv[U][W], av[U][MT];
 #pragma unroll
         for (int q = 0; q < U; q++) {
-            const unsigned p = min(p0 + q * kg, ke - 1);
+            const int p = min(p0 + q * kg, ke - 1);
             if (W == 4)
                 *reinterpret_cast<float4 *>(bv[q]) = *reinterpret_cast<const float4 *>(B + (size_t)p * n);
             else
@@ -405,6 +406,8 @@ __global__ __launch_bounds__(256) void k_mv_cols(const float *__restrict__ a, co
 }
 
 #define LAUNCH_CHECK() SCRY_HIP(hipGetLastError()); return SCRY_OK
+
+constexpr int kHuge = 0x7fffffff - 1024;  // up to here tiles, steps and strides end below 2^31
 
 // parts of p (1 or more) that cover x > 0
 unsigned parts(unsigned x, unsigned p) { return (x + p - 1) / p; }
@@ -464,7 +467,7 @@ int mv_cols(const float *a, const float *b, const float *bias, int batch, int m,
     splits = (int)parts(k, parts(k, splits));  // none empty
     void *ws = nullptr;
     SCRY_TRY(split_workspace(sizeof(double) * (size_t)batch * m * n, &splits, &ws));
-    const unsigned kchunk = parts(k, splits);
+    const int kchunk = (int)parts(k, splits);
     const dim3 g(cb, splits, batch);
     if (W == 4)
         hipLaunchKernelGGL((k_mv_cols<MT, 4>), g, dim3(256), 0, s, a, b, bias, batch, m, k, n, ta, cg, splits, kchunk,
@@ -483,8 +486,8 @@ int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, i
                       const float *bias, float *c, hipStream_t s) {
     if ((size_t)batch * m * n == 0) return SCRY_OK;
     // few rows: reading B is the work and the f64 vector units keep up (the
-    // batch and n limits are the grid's)
-    if (m <= 4 && batch <= 65535 && n <= (1 << 26)) {
+    // batch and n limits are the grid's, k's that of int strides)
+    if (m <= 4 && batch <= 65535 && n <= (1 << 26) && k <= kHuge) {
         if (tb) return m == 1   ? mv_rows<1>(a, b, bias, batch, m, k, n, ta, c, s)
                        : m == 2 ? mv_rows<2>(a, b, bias, batch, m, k, n, ta, c, s)
                                 : mv_rows<4>(a, b, bias, batch, m, k, n, ta, c, s);
@@ -502,13 +505,15 @@ int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, i
     p.k = k;
     p.n = n;
     auto tiles = [&](int t) { return (size_t)batch * parts(m, t) * parts(n, t); };
-    const bool wide = std::max({m, n, k}) > (1 << 21);  // 31-bit offsets: 64 rows of k, or 32 k rows of m or n values
+    const int dim = std::max({m, n, k});
+    const bool huge = dim > kHuge;
+    const bool wide = dim > (1 << 21);  // 31-bit offsets: 64 rows of k, or 32 k rows of m or n values
     // 64 x 64 tiles where they fill the CUs or a long k can be split over
     // them, else 32 x 32 (12 x 200 x 200 x 64: 6 against 14 us; 64 x 4096 x
     // 4096, split: 62 against 49 us).  128 x 128 was slower everywhere
     // (1500 x 1280 x 5120: 513 against 368 us, one wave per SIMD).
     const int steps = (int)parts(k, MM_BK);
-    const int t = tiles(64) >= 256 || (steps >= 64 && m > 32 && n > 32) ? 64 : 32;
+    const int t = huge ? 32 : tiles(64) >= 256 || (steps >= 64 && m > 32 && n > 32) ? 64 : 32;
     p.tm = (int)parts(m, t);
     p.tn = (int)parts(n, t);
     const size_t nt = tiles(t);
@@ -518,7 +523,9 @@ int launch_matmul_f32(const float *a, const float *b, int batch, int m, int k, i
     SCRY_TRY(split_workspace(sizeof(double) * (size_t)batch * m * n, &p.splits, &ws));
     p.part = (double *)ws;
     p.kchunk = parts(steps, p.splits) * MM_BK;
-    if (wide)
+    if (huge)
+        mm_launch<32, LD_HUGE>(p, ta, tb, s);
+    else if (wide)
         t == 32 ? mm_launch<32, LD_WIDE>(p, ta, tb, s) : mm_launch<64, LD_WIDE>(p, ta, tb, s);
     else if (k % 4 == 0)
         t == 32 ? mm_launch<32, LD_QUAD>(p, ta, tb, s) : mm_launch<64, LD_QUAD>(p, ta, tb, s);

@@ -96,7 +96,8 @@ def test_matmul_reads_nothing_past_a_matrix(hip, k, ta, tb):
 TOP = 2 ** 31 - 1  # the largest dimension an entry point takes
 
 
-@pytest.mark.parametrize("m,k,n,tb", [(1, TOP, 1, 1), (1, TOP - 31, 1, 0), (5, TOP, 1, 1), (TOP, 1, 1, 0), (1, 1, TOP, 0)])
+@pytest.mark.parametrize("m,k,n,tb", [(1, TOP, 1, 1), (1, TOP - 1024, 1, 0), (5, TOP, 1, 1), (TOP, 1, 1, 0),
+                                     (1, 1, TOP, 0), (TOP - 1024, 1, 1, 0)])
 def test_matmul_largest_dimension(hip, m, k, n, tb):
     """A dimension whose last tile or stride ends past 2^31 - 1.  Products of
     ones: the f64 sums are exact, so a position left out or taken twice shows."""
